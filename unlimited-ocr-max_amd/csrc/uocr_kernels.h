@@ -86,6 +86,17 @@ hipError_t launch_gemv(const GemvArgs& a, int max_groups, int nproj, int waves, 
 hipError_t launch_gemv_pair(const GemvArgs& routed, int max_groups, const GemvArgs& shared, int nproj,
                             int waves, hipStream_t s);
 
+// The same results on the fp32 matrix instruction, for several rows per weight
+// (gemv_mfma.hip): 16-byte aligned weights and activations, 128-element int8
+// groups, K a multiple of 64 (the _ok checks).
+constexpr int kMfmaWaves = 4;
+bool rows_pair_ok(const GemvArgs& routed, const GemvArgs& shared, int nproj);
+bool rows_routed_ok(const GemvArgs& a);
+bool rows_dense_ok(const GemvArgs& a);
+hipError_t launch_rows_routed(const GemvArgs& a, int max_groups, hipStream_t s);
+hipError_t launch_rows_pair(const GemvArgs& routed, int max_groups, const GemvArgs& shared, int nproj, hipStream_t s);
+hipError_t launch_rows_dense(const GemvArgs& a, hipStream_t s);
+
 // ---- routing (route.hip) ----
 
 // logits[t*E + e] = dot(x[t], router[e]) in the 64-lane tree order; xb (may

@@ -390,7 +390,10 @@ int routed_qmv(const char* op, WKind kind, float* result, const float* x, const 
   }
   a.batch = batch_for(a.nchunks);
   a.rows = rows_of(g);
-  e = launch_gemv(a, max_groups, 1, waves_for(a.batch), s);
+  // Few int8 groups (a token or two) leave most SIMDs without a wave of the matrix path, whose waves take
+  // all chunks of their columns: 6 rows of 64 experts' gate took 16.1 us there and 7.8 us with a wave per
+  // chunk; 18 rows 16.7 against 22.2 us.
+  e = rows_routed_ok(a) && (kind != kInt8Rows || max_groups > 8) ? launch_rows_routed(a, max_groups, s) : launch_gemv(a, max_groups, 1, waves_for(a.batch), s);
   return e == hipSuccess ? 0 : hip_fail(err, errlen, op, e);
 }
 
@@ -492,7 +495,8 @@ int uocr_dense_bf16_qmv(float* result, int64_t result_m, int64_t result_n, const
   a.vec = aligned16(w);
   a.batch = batch_for(a.nchunks);
   a.rows = Rows{nullptr, nullptr, nullptr, nullptr, (int)x_m};
-  const hipError_t e = launch_dense(a, waves_for(a.batch), (hipStream_t)stream);
+  const hipError_t e = rows_dense_ok(a) ? launch_rows_dense(a, (hipStream_t)stream)
+                                        : launch_dense(a, waves_for(a.batch), (hipStream_t)stream);
   return e == hipSuccess ? 0 : hip_fail(err, errlen, "dense_bf16_qmv", e);
 }
 
@@ -1086,7 +1090,8 @@ static int decode_rows_impl(const char* op, float* out, const float* x, int64_t 
   sgu.batch = batch_for(sgu.nchunks);
   sgu.rows = Rows{nullptr, nullptr, nullptr, nullptr, (int)B};
   const int w1 = waves_for(gu.batch > sgu.batch ? gu.batch : sgu.batch);
-  e = launch_gemv_pair(gu, max_groups, sgu, 2, w1, s);
+  e = rows_pair_ok(gu, sgu, 2) ? launch_rows_pair(gu, max_groups, sgu, 2, s)
+                               : launch_gemv_pair(gu, max_groups, sgu, 2, w1, s);
   if (e != hipSuccess) return hip_fail(err, errlen, op, e);
 
   // down for the routed rows and the shared experts
@@ -1121,7 +1126,8 @@ static int decode_rows_impl(const char* op, float* out, const float* x, int64_t 
   sdn.vec = aligned16(L->shared_down);
   sdn.batch = batch_for(sdn.nchunks);
   const int w2 = waves_for(dn.batch > sdn.batch ? dn.batch : sdn.batch);
-  e = launch_gemv_pair(dn, max_groups, sdn, 1, w2, s);
+  e = rows_pair_ok(dn, sdn, 1) ? launch_rows_pair(dn, max_groups, sdn, 1, s)
+                               : launch_gemv_pair(dn, max_groups, sdn, 1, w2, s);
   if (e == hipSuccess) e = launch_combine(out, d.y, H, d.wts, nullptr, d.sh, (int)B, H, (int)L->top_k, s);
   if (e == hipSuccess && expert_ids) e = hipMemcpyAsync(expert_ids, d.ids, R * sizeof(int32_t), hipMemcpyDeviceToDevice, s);
   if (e == hipSuccess && expert_weights)
