@@ -625,16 +625,23 @@ hipError_t launch_moe_gemm(const GemmProblem& routed, const GemmProblem& shared,
 // work, about ten VALU instructions per MFMA, bounds a lone wave).  A step is
 // 64 k: every weight row contributes 64 (int8) or 128 (bf16) contiguous bytes,
 // 4 or 8 lanes to a row, where the fragment-layout loads touch 32 rows per
-// instruction.  A stage holds the workgroup's 256 weight rows and the A step;
-// kCount stages form a ring, each loaded kCount - 1 steps ahead.  The int8
-// scales of the tile's weight rows (one contiguous block of rows x groups
+// instruction.  Weights and A steps lie in two rings of LDS slots (Ring), each
+// loaded a slot less than its depth ahead.  The int8 scales of the tile's
+// weight rows (one contiguous block of rows x groups
 // floats per projection) are loaded into LDS once, at the tile's start: read
 // step by step they would touch a cache line per few rows every step.  The
 // waits are explicit (s_waitcnt vmcnt(n) before the barrier, n the loads
 // issued since the step's own): every thread issues the same number of loads
-// per step, the loads past the last step re-read it, and no other vector
+// per step and no other vector
 // memory access happens inside the K loop.  Lane half h covers k = 32h ..
 // 32h + 31 of a step, as in the fragment-load path, so both give the same bits.
+//
+// What bounds the K loop is its issue: a 128-row int8 step is 32 MFMAs and
+// about 170 VALU instructions a wave, and a wave issues in order.  With the
+// dequantisation one sub-step ahead and spread between the MFMAs, and the
+// loads' addresses scalar (a uniform base plus a lane offset: 22 VALU less a
+// step), T = 4096 gate/up takes 193 us where the compiler's own order (bursts
+// of both) took 217; with the third weight slot T = 512 takes 54 us for 56.
 
 // Rows per tile of the LDS-staged path: 128 for int8 weights (each
 // dequantised weight feeds up to four 32-row MFMA blocks; blocks past a
@@ -654,22 +661,29 @@ struct Stage {
   static constexpr int kBRowBytes = W == kInt8Rows ? BK : 2 * BK;  // one step of a weight row
   static constexpr int kBBytes = kWRowsWg * kBRowBytes;
   static constexpr int kABytes = BM * 2 * BK;
-  static constexpr int kBytes = kBBytes + kABytes;
   static constexpr int kBudget = 160 * 1024 / kWgPerCu - (W == kInt8Rows ? kScaleLds : 0);
-  static constexpr int kCount = kBudget / kBytes < 4 ? kBudget / kBytes : 4;
   static constexpr int kBLoads = kBBytes / 1024 / 4;  // weight loads per thread per step
-  // loads per thread per step of a tile with NACT active 32-row blocks: the
-  // weights and one 1 KB A load per block (32 rows x 128 bytes over 256 threads)
-  template <int NACT>
-  static constexpr int loads() {
-    return kBLoads + NACT;
-  }
-  static_assert(kCount >= 2, "two stages");
+  static_assert(2 * (kBBytes + kABytes) <= kBudget, "two stages of a full tile");
   static_assert(kABytes == (BM / 32) * 16 * kGThreads, "one A load per thread per 32-row block");
 };
 
+// The rings of a tile with NACT active 32-row blocks: kB slots of weights, then
+// kA slots of the active blocks' A rows, in the bytes two full stages take.  A
+// tile of few rows leaves room for a third weight slot (and, at one block, a
+// third A slot): its steps are short and wait on memory, so a second step of
+// weights in flight is what they lack.
+template <int BM, WKind W, int NACT>
+struct Ring {
+  using St = Stage<BM, W>;
+  static constexpr int kAStep = NACT * 32 * 2 * BK;  // one step's A bytes
+  static constexpr int kBytes = 2 * (St::kBBytes + St::kABytes);
+  static constexpr int kB = 3 * St::kBBytes + 2 * kAStep <= kBytes ? 3 : 2;
+  static constexpr int kA = kB * (St::kBBytes + kAStep) <= kBytes ? kB : 2;
+  static constexpr int kALoads = NACT;  // A loads per thread per step: 32 rows x 128 bytes over 256 threads
+};
+
 template <WKind W>
-constexpr int kRing = Stage<kLdsBM<W>, W>::kBytes * Stage<kLdsBM<W>, W>::kCount;
+constexpr int kRing = Ring<kLdsBM<W>, W, kLdsBM<W> / 32>::kBytes;
 template <WKind W>
 constexpr int kTileLds = kRing<W> + (W == kInt8Rows ? kScaleLds : 0);  // the scales follow the ring
 template <WKind W0>
@@ -678,6 +692,13 @@ constexpr int kLdsBytes = kTileLds<W0> > kTileLds<kBf16KBlocked> ? kTileLds<W0> 
 typedef __attribute__((address_space(3))) void* lds_ptr;
 __device__ __forceinline__ void dma16(const void* g, void* l) {
   __builtin_amdgcn_global_load_lds((const UOCR_GLOBAL void*)g, (lds_ptr)l, 16, 0, 0);
+}
+// A lane offset for dma16(uniform base + offset), made opaque (in place) where
+// it is used: the compiler then takes the load's own base + 32-bit offset form
+// and does not keep (or add up) 64-bit lane addresses.
+__device__ __forceinline__ uint32_t lane_offset(uint32_t& off) {
+  asm volatile("" : "+v"(off));
+  return off;
 }
 __device__ __forceinline__ void dma4(const void* g, void* l) {
   __builtin_amdgcn_global_load_lds((const UOCR_GLOBAL void*)g, (lds_ptr)l, 4, 0, 0);
@@ -702,14 +723,13 @@ __device__ __forceinline__ int swz64(int r) { return ((r >> 1) & 3) ^ ((r >> 3) 
 // computed).  The wave's weight bytes of the step are read first, and the A
 // fragments of sub-step k + 1 before the MFMAs of sub-step k.
 template <int BM, WKind W, int NACT>
-__device__ __forceinline__ void lds_step(f32x16 (&acc)[NACT][2], const char* st, const float (&sc)[2], int w, int m,
-                                         int h) {
+__device__ __forceinline__ void lds_step(f32x16 (&acc)[NACT][2], const char* st, const char* A, const float (&sc)[2],
+                                         int w, int m, int h) {
   using St = Stage<BM, W>;
   constexpr int MB = NACT;
   constexpr int RB = St::kBRowBytes;
   constexpr int NQ = W == kInt8Rows ? 2 : 4;  // the lane's 16-byte weight chunks per block
   const char* Bw = st + 64 * w * RB;          // the wave's 64 weight rows
-  const char* A = st + St::kBBytes;
   const int sw = swz(m);  // 128-byte rows 32i + m (A, bf16 weights)
   i32x4 raw[2][NQ];
 #pragma unroll
@@ -726,41 +746,65 @@ __device__ __forceinline__ void lds_step(f32x16 (&acc)[NACT][2], const char* st,
         raw[b][q] = *(const i32x4*)(Bw + (32 * b + m) * RB + 16 * (c ^ (W == kInt8Rows ? swz64(m) : sw)));
       }
     }
-  // The A fragments of sub-step k + 1 are read during sub-step k.
-  constexpr int AB = 2;
-  bf16x8 a[AB][MB];
+  // The step's B fragments as 32 dwords, n = 8 sub + 4 b + d: convert(n) makes
+  // dword n's two weights floats, finish(n) scales and packs them.
+  float q[2];
+  auto convert = [&](int n) {
+    if constexpr (W == kInt8Rows) {
+      const int sub = n >> 3, b = (n >> 2) & 1, d = n & 3;
+      const int v = raw[b][sub >> 1][(sub & 1) * 2 + (d >> 1)];
+      q[0] = (d & 1) ? i8_to_f32<2>(v) : i8_to_f32<0>(v);
+      q[1] = (d & 1) ? i8_to_f32<3>(v) : i8_to_f32<1>(v);
+    }
+  };
+  auto finish = [&](int n) -> int {
+    const int sub = n >> 3, b = (n >> 2) & 1, d = n & 3;
+    if constexpr (W == kInt8Rows)
+      return (int)pack_bf16x2(q[0] * sc[b], q[1] * sc[b]);
+    else
+      return raw[b][sub][d];
+  };
+  bf16x8 a[2][MB];
+  i32x4 bw[2][2];
   auto read_a = [&](bf16x8(&dst)[MB], int sub) {
 #pragma unroll
     for (int i = 0; i < MB; ++i) dst[i] = *(const bf16x8*)(A + (32 * i + m) * 2 * BK + 16 * ((4 * h + sub) ^ sw));
   };
-  if constexpr (AB == 2) read_a(a[0], 0);
+  read_a(a[0], 0);
+#pragma unroll
+  for (int n = 0; n < 8; ++n) {
+    convert(n);
+    bw[0][n >> 2][n & 3] = finish(n);
+  }
+  convert(8);
+  if (W == kInt8Rows) __builtin_amdgcn_sched_barrier(0);
+  // The A fragments and the dequantised weights of sub-step k + 1 are made
+  // ready during sub-step k, the dequantisation spread between the MFMAs in
+  // program order: a wave issues in order, so a VALU instruction behind two
+  // MFMAs waits for the first, while a dword's five fit under one.  A dword's
+  // conversions come a slot ahead of its products (read at once, they cost a
+  // wait state).
 #pragma unroll
   for (int sub = 0; sub < 4; ++sub) {
-    if constexpr (AB == 2) {
-      if (sub < 3) read_a(a[(sub + 1) & 1], sub + 1);
-    } else {
-      read_a(a[0], sub);
-    }
-    bf16x8 bf[2];
+    const int c = sub & 1;
+    if (sub < 3) read_a(a[c ^ 1], sub + 1);
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      if constexpr (W == kInt8Rows) {
-        const int d0 = raw[b][sub >> 1][(sub & 1) * 2], d1 = raw[b][sub >> 1][(sub & 1) * 2 + 1];
-        i32x4 o;
-        o[0] = (int)pack_bf16x2(i8_to_f32<0>(d0) * sc[b], i8_to_f32<1>(d0) * sc[b]);
-        o[1] = (int)pack_bf16x2(i8_to_f32<2>(d0) * sc[b], i8_to_f32<3>(d0) * sc[b]);
-        o[2] = (int)pack_bf16x2(i8_to_f32<0>(d1) * sc[b], i8_to_f32<1>(d1) * sc[b]);
-        o[3] = (int)pack_bf16x2(i8_to_f32<2>(d1) * sc[b], i8_to_f32<3>(d1) * sc[b]);
-        bf[b] = __builtin_bit_cast(bf16x8, o);
-      } else {
-        bf[b] = __builtin_bit_cast(bf16x8, raw[b][sub]);
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        acc[i][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[c][i], __builtin_bit_cast(bf16x8, bw[c][b]), acc[i][b],
+                                                            0, 0, 0);
+        if (sub < 3) {
+          const int u = 2 * i + b;  // MFMA u of 2 MB covers dwords [8 u / (2 MB), 8 (u + 1) / (2 MB))
+#pragma unroll
+          for (int d = 8 * u / (2 * MB); d < 8 * (u + 1) / (2 * MB); ++d) {
+            const int n = 8 * (sub + 1) + d;
+            bw[c ^ 1][d >> 2][d & 3] = finish(n);
+            if (n + 1 < 32) convert(n + 1);
+          }
+        }
+        if (W == kInt8Rows) __builtin_amdgcn_sched_barrier(0);
       }
-    }
-#pragma unroll
-    for (int i = 0; i < MB; ++i) {
-      acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[sub % AB][i], bf[0], acc[i][0], 0, 0, 0);
-      acc[i][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[sub % AB][i], bf[1], acc[i][1], 0, 0, 0);
-    }
   }
 }
 
@@ -769,8 +813,8 @@ __device__ __forceinline__ void lds_step(f32x16 (&acc)[NACT][2], const char* st,
 template <int BM, WKind W, int NPROJ, int NACT>
 __device__ __forceinline__ void lds_tile(const GemmProblem& P, const TileRef& t, char* lds) {
   using St = Stage<BM, W>;
-  constexpr int NS = St::kCount, NB = St::kBLoads, NA = NACT;
-  constexpr int NL = St::template loads<NACT>();
+  using Rg = Ring<BM, W, NACT>;
+  constexpr int NB = St::kBLoads, NA = Rg::kALoads, NL = NB + NA;
   constexpr int RB = St::kBRowBytes;
   constexpr int RPL = 1024 / RB;  // weight rows per load
   // The thread index passes through an empty asm per tile, so that what is
@@ -781,7 +825,7 @@ __device__ __forceinline__ void lds_tile(const GemmProblem& P, const TileRef& t,
   int tid = (int)threadIdx.x;
   asm volatile("" : "+v"(tid));
   const int j = tid & (kWave - 1);
-  const int w = tid >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = j & 31, h = j >> 5;
   // the tile's K range: all of K, or range t.e of a problem in K ranges
   const int parts = parts_of(P);
@@ -789,8 +833,10 @@ __device__ __forceinline__ void lds_tile(const GemmProblem& P, const TileRef& t,
   const int k0 = parts > 1 ? t.e * S : 0;
 
   // weight rows: load i of the step fills stage rows 64w + RPL i + j / (RB / 16),
-  // stored chunk j % (RB / 16) holding chunk (stored) ^ swizzle(row)
-  const char* bsrc[NB];
+  // stored chunk j % (RB / 16) holding chunk (stored) ^ swizzle(row).  A load's
+  // address is a wave-uniform base (expert, projection, first column, step) plus
+  // the lane's 32-bit offset, so a step's loads take no vector arithmetic.
+  uint32_t boff[NB];
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
     if constexpr (W == kBf16KBlocked) {
@@ -798,36 +844,33 @@ __device__ __forceinline__ void lds_tile(const GemmProblem& P, const TileRef& t,
       // 1 KB contiguous in [K/16][N][16]; lane j holds half (j % 2) ^ (row bit 3) of row j / 2
       const int b = i & 1;
       const int lr = j >> 1;
-      const int row = min(NPROJ == 2 ? t.n0 + 32 * w + lr : t.n0 + 64 * w + 32 * b + lr, P.N - 1);
+      const int row = min(NPROJ == 2 ? 32 * w + lr : 64 * w + 32 * b + lr, P.N - 1 - t.n0);
       const int hf = (j & 1) ^ ((lr >> 3) & 1);
-      const char* base = (const char*)(NPROJ == 2 && b == 1 ? P.p[1].w : P.p[0].w);
-      bsrc[i] = base + ((int64_t)(i >> 1) * P.N + row) * 32 + 16 * hf;
+      boff[i] = (uint32_t)(row * 32 + 16 * hf);
       continue;
     }
     const int rr = RPL * i + j / (RB / 16);  // row within the wave's 64
-    const int b = rr >> 5;
     const int mm = rr & 31;
-    const int row = min(NPROJ == 2 ? t.n0 + 32 * w + mm : t.n0 + 64 * w + rr, P.N - 1);
+    const int row = min(NPROJ == 2 ? 32 * w + mm : 64 * w + rr, P.N - 1 - t.n0);
     const int c = (j % (RB / 16)) ^ (W == kInt8Rows ? swz64(rr) : swz(rr));
-    const char* base = (const char*)(NPROJ == 2 && b == 1 ? P.p[1].w : P.p[0].w);
-    const int64_t wrow = (int64_t)t.e * P.N + row;
-    if constexpr (W == kInt8Rows)
-      bsrc[i] = base + wrow * P.K + 16 * c;
-    else
-      bsrc[i] = base + wrow * P.K * 2 + 16 * c;
+    boff[i] = (uint32_t)(row * RB * (P.K / BK) + 16 * c);
   }
   const int64_t bstep = W == kBf16KBlocked ? (int64_t)(BK / 16) * P.N * 32 : RB;
+  const int64_t bfirst = W == kBf16KBlocked ? (int64_t)t.n0 * 32
+                                            : ((int64_t)t.e * P.N + t.n0) * RB * (P.K / BK);
+  // load i's projection: block 1 of the wave's 64 rows is up in a gate/up launch
+  constexpr auto up_load = [](int i) { return NPROJ == 2 && (W == kBf16KBlocked ? i & 1 : RPL * i >= 32); };
 
   // A: load i of the step fills 1 KB unit 4i + w of the A stage, chunk j % 8 of
   // stage row 8 (4i + w) + j / 8
-  int aoff[NA];
+  uint32_t aoff[NA];
 #pragma unroll
   for (int i = 0; i < NA; ++i) {
     const int r = 8 * (4 * i + w) + (j >> 3);
     const int c = (j & 7) ^ swz(r);
     const int pos = t.pos0 + min(r, t.rows - 1);
     const int row = (P.a_by_token && P.rows.n_groups != nullptr) ? ldg(P.rows.group_rows + pos) / P.x_div : pos;
-    aoff[i] = (int)((int64_t)row * P.lda) + 8 * c;
+    aoff[i] = 2u * ((uint32_t)((int64_t)row * P.lda) + 8u * c);
   }
 
   // int8 scales, loaded once for the tile after the ring: NPROJ 1, [256 rows
@@ -852,19 +895,25 @@ __device__ __forceinline__ void lds_tile(const GemmProblem& P, const TileRef& t,
   }
   const int spg = W == kInt8Rows ? P.K / P.groups / BK : 1;  // steps per scale group
 
-  // the loads of step s (clamped to the last step) into stage s % NS
-  auto issue = [&](int s) {
-    const int sc = k0 + min(s, S - 1);
-    char* st = lds + (s % NS) * St::kBytes;
+  // the weight (A) loads of step s into slot s % kB (s % kA) of their ring
+  auto issue_b = [&](int s) {
+    char* st = lds + (s % Rg::kB) * St::kBBytes;
+    const int64_t at = bfirst + (k0 + s) * bstep;
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
+      const char* base = (const char*)(up_load(i) ? P.p[1].w : P.p[0].w) + at;
+      const uint32_t off = lane_offset(boff[i]);
       if constexpr (W == kBf16KBlocked)
-        dma16(bsrc[i] + sc * bstep, st + ((i >> 1) * kWRowsWg + 64 * w + 32 * (i & 1)) * 32);
+        dma16(base + (int64_t)(i >> 1) * P.N * 32 + off, st + ((i >> 1) * kWRowsWg + 64 * w + 32 * (i & 1)) * 32);
       else
-        dma16(bsrc[i] + sc * bstep, st + (64 * w + RPL * i) * RB);
+        dma16(base + off, st + (64 * w + RPL * i) * RB);
     }
+  };
+  auto issue_a = [&](int s) {
+    char* st = lds + Rg::kB * St::kBBytes + (s % Rg::kA) * Rg::kAStep;
+    const char* base = (const char*)(P.a + (k0 + s) * BK);
 #pragma unroll
-    for (int i = 0; i < NA; ++i) dma16(P.a + aoff[i] + sc * BK, st + St::kBBytes + (4 * i + w) * 1024);
+    for (int i = 0; i < NA; ++i) dma16(base + lane_offset(aoff[i]), st + (4 * i + w) * 1024);
   };
 
   f32x16 acc[NACT][2];
@@ -882,30 +931,36 @@ __device__ __forceinline__ void lds_tile(const GemmProblem& P, const TileRef& t,
       g += next;
       gs = next ? 0 : gs;
     }
-    lds_step<BM, W, NACT>(acc, lds + (s % NS) * St::kBytes, sc, w, m, h);
+    lds_step<BM, W, NACT>(acc, lds + (s % Rg::kB) * St::kBBytes,
+                          lds + Rg::kB * St::kBBytes + (s % Rg::kA) * Rg::kAStep, sc, w, m, h);
   };
-  // S is even and at least 2, so the NS - 1 <= 2 prologue steps exist; the
-  // last NS - 1 steps load nothing, and no load is in flight when the tile ends
-  static_assert(NS >= 2 && NS <= 3, "ring depth");
+  // Step s issues the A loads of step s + LA, then the weight loads of step s +
+  // LB (LA = LB, or LB - 1); so when it starts, the loads after its own A are
+  // the weights of one step (LA < LB) and LA - 1 whole steps.  S is even and at
+  // least 2, so the prologue's steps exist; the last LB steps load no weights,
+  // and no load is in flight when the tile ends.
+  constexpr int LA = Rg::kA - 1, LB = Rg::kB - 1;
+  static_assert(LA >= 1 && LB <= 2 && (LA == LB || LA == LB - 1), "ring depth");
 #pragma unroll
-  for (int i = 0; i < NS - 1; ++i) issue(i);
-  for (int s = 0; s < S - (NS - 1); ++s) {
-    step_barrier<(NS - 2) * NL>();
-    issue(s + NS - 1);  // into the stage read in step s - 1, which every wave has finished
+  for (int i = -LB; i < 0; ++i) {
+    if (i + LA >= 0) issue_a(i + LA);
+    issue_b(i + LB);
+  }
+  for (int s = 0; s < S - LB; ++s) {
+    step_barrier<(LB - LA) * NB + (LA - 1) * NL>();
+    issue_a(s + LA);  // into slots read in step s - 1, which every wave has finished
+    issue_b(s + LB);
     compute(s);
   }
 #pragma unroll
-  for (int u = 0; u < NS - 1; ++u) {
-    // tail step S - (NS - 1) + u: its loads and the NS - 2 - u stages after it are the ones outstanding
-    if constexpr (NS == 3) {
-      if (u == 0)
-        step_barrier<NL>();
-      else
-        step_barrier<0>();
-    } else {
+  for (int u = 0; u < LB; ++u) {
+    const int s = S - LB + u;
+    if (u + 1 == LB)
       step_barrier<0>();
-    }
-    compute(S - (NS - 1) + u);
+    else
+      step_barrier<(LB - LA) * NB + (LA - 1) * NL>();
+    if (LA < LB && u + 1 < LB) issue_a(s + LA);
+    compute(s);
   }
   // every wave has finished reading the stages (and the scales) before the next tile's loads
   step_barrier<0>();
