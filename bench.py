@@ -654,16 +654,12 @@ def _by_name(part: str) -> Callable[[list], list]:
 
 
 def prefill_gemm_dispatches(rows: list) -> dict[str, list]:
-    """The prefill probe's GEMM dispatches by workload, in its launch order: T=512 over the 11 layers, then
-    T=4096 and the adversarial T=4096 over 4 layers each; gate/up and down alternate within a layer."""
-    gemms = [r for r in rows if "k_moe_gemm" in r[1]]
-    n512, n4k = 2 * LAYERS, 2 * PREFILL_4K_LAYERS
-    groups = {"t512": gemms[:n512], "t4096": gemms[n512:n512 + n4k], "t4096_adversarial": gemms[n512 + n4k:]}
-    out = {}
-    for name, g in groups.items():
-        out[f"{name}_gateup"] = g[0::2]
-        out[f"{name}_down"] = g[1::2]
-    return out
+    """The prefill probe's GEMM dispatches (gate/up and down in one) by workload, in its launch order: T=512
+    over the 11 layers, then T=4096 and the adversarial T=4096 over 4 layers each."""
+    gemms = [r for r in rows if "k_moe_layer" in r[1]]
+    n512, n4k = LAYERS, PREFILL_4K_LAYERS
+    return {"t512_gemm": gemms[:n512], "t4096_gemm": gemms[n512:n512 + n4k],
+            "t4096_adversarial_gemm": gemms[n512 + n4k:]}
 
 
 def prefill_probe() -> int:
@@ -837,7 +833,7 @@ def main() -> int:
                 r = results.get(key)
                 if r is None:
                     continue
-                for kind, kname in (("gateup", "gemm_gateup"), ("down", "gemm_down")):
+                for kind, kname in (("gemm", "gemm_layer"),):
                     c = pc.get(f"{label}_{kind}")
                     us = r["kernels_us_avg"].get(kname)
                     if c is None or us is None:
@@ -846,7 +842,7 @@ def main() -> int:
                     c["mfma_tflops_executed"] = round(c["mfma_flops_per_launch"] / (us * 1e-6) / 1e12, 1)
                     if "traffic_bytes" in c:
                         c["traffic_gbs"] = round(c["traffic_bytes"] / (us * 1e-6) / 1e9, 1)
-                r["mfma_busy_frac"] = {k: pc[f"{label}_{k}"]["mfma_busy_frac"] for k in ("gateup", "down")
+                r["mfma_busy_frac"] = {k: pc[f"{label}_{k}"]["mfma_busy_frac"] for k in ("gemm",)
                                        if f"{label}_{k}" in pc}
     line = {
         "metric": METRIC,

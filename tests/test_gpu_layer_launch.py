@@ -1,0 +1,111 @@
+"""The prefill layer's one GEMM launch (gate/up tiles, then down tiles that wait for their rows).
+
+Weights at an odd address take the fragment-load kernel, a launch per phase and the same bits, so the two
+paths are compared bit for bit: at the edges of the tiles (32-row blocks, 64- and 128-row tiles), with one
+expert or more tiles than workgroups, and as the launch meets itself: replayed, and on two streams at once.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from _gpu import DEV, bits_equal, layer_weights, moe_for, n, t
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {  # experts, hidden, ffn (top 2, 2 shared experts)
+    "small": (8, 256, 128),
+    "many": (64, 256, 256),
+    "one": (1, 128, 128),
+}
+
+
+def _pair(oracle, shape: str, int8: bool):
+    """A layer with aligned weights, and the same one with its gate stack at an odd (2-byte for bf16) address."""
+    from uocr_moe import MoE
+
+    E, H, F = SHAPES[shape]
+    layer = oracle.make_layer(5, E=E, H=H, F=F, topk=min(2, E), int8=int8, std=0.05, router_std=0.1)
+    moe = moe_for(layer)
+    w = layer_weights(layer)
+    gate = w["experts.gate_proj"]
+    raw = torch.empty(gate.numel() * gate.element_size() + 16, dtype=torch.uint8, device=DEV)
+    off = gate.element_size()
+    odd = raw[off:off + gate.numel() * gate.element_size()].view(gate.dtype).view(gate.shape)
+    odd.copy_(gate)
+    w["experts.gate_proj"] = odd
+    other = MoE(moe.config, w)
+    assert other.stacks["gate_proj"].data_ptr() % 16 != 0
+    return moe, other
+
+
+def _x(T: int, H: int) -> torch.Tensor:
+    return t(np.random.default_rng(T).standard_normal((T, H)).astype(np.float32))
+
+
+@pytest.mark.parametrize("int8", [True, False])
+@pytest.mark.parametrize(("shape", "T"), [("one", 1), ("one", 64), ("one", 129), ("one", 300), ("small", 1),
+                                          ("small", 31), ("small", 130), ("small", 515), ("many", 65),
+                                          ("many", 2049), ("many", 6000)])
+def test_one_launch_is_the_two(oracle, shape, T, int8) -> None:
+    moe, other = _pair(oracle, shape, int8)
+    x = _x(T, SHAPES[shape][1])
+    assert bits_equal(n(moe(x)), n(other(x)))
+
+
+def test_many_down_tiles(oracle) -> None:
+    """Few gate/up tiles and more down tiles than the by-class plan holds."""
+    from uocr_moe import MoE, MoeConfig
+
+    E, H, F, T = 64, 4608, 128, 2048
+    g = torch.Generator(device=DEV).manual_seed(1)
+
+    def w(*shape: int) -> torch.Tensor:
+        return (torch.randn(shape, generator=g, device=DEV) * 0.05).to(torch.bfloat16)
+
+    weights = {"gate.gate_score.weight": w(E, H).float(), "experts.gate_proj": w(E, F, H),
+               "experts.up_proj": w(E, F, H), "experts.down_proj": w(E, H, F),
+               "shared_experts.gate_proj.weight": w(H // 16, 2 * F, 16),
+               "shared_experts.up_proj.weight": w(H // 16, 2 * F, 16),
+               "shared_experts.down_proj.weight": w(2 * F // 16, H, 16)}
+    config = MoeConfig(hidden_size=H, moe_intermediate_size=F, n_routed_experts=E, num_experts_per_tok=1,
+                       n_shared_experts=2, int8_experts=False)
+    x = _x(T, H)
+    got = n(MoE(config, weights)(x))
+    raw = torch.empty(E * F * H + 8, dtype=torch.bfloat16, device=DEV)
+    odd = raw[1:1 + E * F * H].view(E, F, H)
+    odd.copy_(weights["experts.gate_proj"])
+    assert bits_equal(got, n(MoE(config, {**weights, "experts.gate_proj": odd})(x)))
+
+
+def test_replays_and_streams(oracle) -> None:
+    """A captured layer replayed between eager calls, then calls on two streams at once."""
+    moe, _ = _pair(oracle, "many", True)
+    xs = [_x(T, 256) for T in (700, 1900)]
+    want = [n(moe(x)) for x in xs]
+    side = torch.cuda.Stream()
+    ws = moe.workspace(700, True)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        moe(xs[0], workspace=ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = moe(xs[0], workspace=ws)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        assert bits_equal(n(moe(xs[1])), want[1])
+        assert bits_equal(n(out), want[0])
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    got: list[list[torch.Tensor]] = [[], []]
+    torch.cuda.synchronize()
+    for _ in range(8):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                got[i].append(moe(xs[i]))
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(bits_equal(n(o), want[i]) for o in got[i])

@@ -18,6 +18,7 @@
 // SIMD -- a second wave does not overlap them -- so the int8 kernels are
 // bounded by that issue time; the tiles are sized to spread each dequantised
 // weight over as many rows as the expert has (up to 128).
+#include <algorithm>
 #include <atomic>
 
 #include "uocr_device.h"
@@ -152,6 +153,8 @@ struct TileRef {
   int pos0;  // first row position (group order) or first token
   int rows;  // valid rows
   int n0;    // first output column
+  int dep;   // its h rows' counter of finished gate/up tiles (k_moe_layer)
+  int need;  // finished gate/up tiles a down tile waits for
 };
 
 // K ranges of a problem (a dense K-blocked one may be cut into kparts).
@@ -467,7 +470,9 @@ __device__ __forceinline__ void quad_transpose(float (&v)[4], int qd) {
 // MFMA layout needs four (scattered 2- and 4-byte stores took 20-30 k cycles a
 // 256 x 256 tile and slowed the loads queued behind them).  Gate/up: h rows in
 // bf16, silu(gate) * up of the two blocks; down: fp32 rows.
-template <int BM, int NPROJ>
+// PUBLISH: h goes past the L2 (agent scope), for down tiles on other XCDs in
+// the same launch.
+template <int BM, int NPROJ, bool PUBLISH = false>
 __device__ __forceinline__ void store_tile(const GemmProblem& P, const TileRef& t, const f32x16 (&acc)[BM / 32][2],
                                            int w, int m, int h) {
   const int qd = m & 3;
@@ -486,7 +491,11 @@ __device__ __forceinline__ void store_tile(const GemmProblem& P, const TileRef& 
         const int col = t.n0 + 32 * w + (m & ~3);
         if (live && col < P.N) {
           const uint64_t o = (uint64_t)pack_bf16x2(v[0], v[1]) | ((uint64_t)pack_bf16x2(v[2], v[3]) << 32);
-          *(UOCR_GLOBAL uint64_t*)(P.outb + orow * P.ldo + col) = o;
+          UOCR_GLOBAL uint64_t* dst = (UOCR_GLOBAL uint64_t*)(P.outb + orow * P.ldo + col);
+          if constexpr (PUBLISH)
+            __hip_atomic_store(dst, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          else
+            *dst = o;
         }
       } else {
 #pragma unroll
@@ -690,8 +699,10 @@ template <WKind W0>
 constexpr int kLdsBytes = kTileLds<W0> > kTileLds<kBf16KBlocked> ? kTileLds<W0> : kTileLds<kBf16KBlocked>;
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
+constexpr int kAgentLoad = 16;  // the load's sc1 bit: agent scope, past the L2
+template <int AUX = 0>
 __device__ __forceinline__ void dma16(const void* g, void* l) {
-  __builtin_amdgcn_global_load_lds((const UOCR_GLOBAL void*)g, (lds_ptr)l, 16, 0, 0);
+  __builtin_amdgcn_global_load_lds((const UOCR_GLOBAL void*)g, (lds_ptr)l, 16, 0, AUX);
 }
 // A lane offset for dma16(uniform base + offset), made opaque (in place) where
 // it is used: the compiler then takes the load's own base + 32-bit offset form
@@ -808,10 +819,26 @@ __device__ __forceinline__ void lds_step(f32x16 (&acc)[NACT][2], const char* st,
   }
 }
 
+constexpr int kCtlLine = 32;  // words between control words
+// The control words of a tile (below): its list's ticket counter, and the
+// finished gate/up tiles.
+struct PhaseCtl {
+  int32_t* ticket;
+  int32_t* done;
+};
+__device__ __forceinline__ int32_t agent_load(const int32_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int32_t agent_add(int32_t* p, int32_t v) {
+  return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 // One tile whose rows fill NACT 32-row blocks: only those blocks' A rows are
-// loaded and computed.
+// loaded and computed.  A gate/up tile (NPROJ 2) counts itself finished once
+// its h rows are past the L2; a down tile waits for its h rows after its first
+// weights are on their way.  Returns the workgroup's next ticket of the list,
+// taken during the last step.
 template <int BM, WKind W, int NPROJ, int NACT>
-__device__ __forceinline__ void lds_tile(const GemmProblem& P, const TileRef& t, char* lds) {
+__device__ __forceinline__ int lds_tile(const GemmProblem& P, const TileRef& t, char* lds, const PhaseCtl& ctl) {
   using St = Stage<BM, W>;
   using Rg = Ring<BM, W, NACT>;
   constexpr int NB = St::kBLoads, NA = Rg::kALoads, NL = NB + NA;
@@ -913,7 +940,7 @@ __device__ __forceinline__ void lds_tile(const GemmProblem& P, const TileRef& t,
     char* st = lds + Rg::kB * St::kBBytes + (s % Rg::kA) * Rg::kAStep;
     const char* base = (const char*)(P.a + (k0 + s) * BK);
 #pragma unroll
-    for (int i = 0; i < NA; ++i) dma16(base + lane_offset(aoff[i]), st + (4 * i + w) * 1024);
+    for (int i = 0; i < NA; ++i) dma16<NPROJ == 1 ? kAgentLoad : 0>(base + lane_offset(aoff[i]), st + (4 * i + w) * 1024);
   };
 
   f32x16 acc[NACT][2];
@@ -941,10 +968,18 @@ __device__ __forceinline__ void lds_tile(const GemmProblem& P, const TileRef& t,
   // and no load is in flight when the tile ends.
   constexpr int LA = Rg::kA - 1, LB = Rg::kB - 1;
   static_assert(LA >= 1 && LB <= 2 && (LA == LB || LA == LB - 1), "ring depth");
+  issue_b(0);
+  if constexpr (NPROJ == 1) {
+    // The wait ends: every gate/up tile has been taken by a running workgroup,
+    // and none of those waits for anything.
+    if (threadIdx.x == 0)
+      while (agent_load(ctl.done + t.dep * kCtlLine) < t.need) __builtin_amdgcn_s_sleep(1);
+    asm volatile("s_barrier" ::: "memory");
+  }
 #pragma unroll
   for (int i = -LB; i < 0; ++i) {
     if (i + LA >= 0) issue_a(i + LA);
-    issue_b(i + LB);
+    if (i > -LB) issue_b(i + LB);
   }
   for (int s = 0; s < S - LB; ++s) {
     step_barrier<(LB - LA) * NB + (LA - 1) * NL>();
@@ -952,6 +987,7 @@ __device__ __forceinline__ void lds_tile(const GemmProblem& P, const TileRef& t,
     issue_b(s + LB);
     compute(s);
   }
+  int ticket = 0;
 #pragma unroll
   for (int u = 0; u < LB; ++u) {
     const int s = S - LB + u;
@@ -960,17 +996,25 @@ __device__ __forceinline__ void lds_tile(const GemmProblem& P, const TileRef& t,
     else
       step_barrier<(LB - LA) * NB + (LA - 1) * NL>();
     if (LA < LB && u + 1 < LB) issue_a(s + LA);
+    if (u + 1 == LB && threadIdx.x == 0) ticket = agent_add(ctl.ticket, 1);
     compute(s);
   }
   // every wave has finished reading the stages (and the scales) before the next tile's loads
   step_barrier<0>();
+  if (threadIdx.x == 0) *(int*)lds = ticket;
   if (parts > 1) {
     GemmProblem Q = P;  // range t.e's sums
     Q.outf += t.e * P.part_stride;
     store_tile<32 * NACT, NPROJ>(Q, t, acc, w, m, h);
   } else {
-    store_tile<32 * NACT, NPROJ>(P, t, acc, w, m, h);
+    store_tile<32 * NACT, NPROJ, NPROJ == 2>(P, t, acc, w, m, h);
   }
+  if constexpr (NPROJ == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // h is past the L2
+  lds_barrier();
+  ticket = __builtin_amdgcn_readfirstlane(*(const int*)lds);
+  if (NPROJ == 2 && threadIdx.x == 0) (void)agent_add(ctl.done + t.dep * kCtlLine, 1);
+  lds_barrier();
+  return ticket;
 }
 
 // Placement for the LDS-staged path, two ways, chosen per launch from the
@@ -983,8 +1027,7 @@ __device__ __forceinline__ void lds_tile(const GemmProblem& P, const TileRef& t,
 // estimated cost (a tile belongs to the range its cost midpoint falls in),
 // range x going to XCD x; the shared experts' row tiles are cut into 8 runs
 // of equal length (all their column tiles), run x going to XCD x ahead of
-// its routed range.  Workgroup j of an XCD walks tiles j, j + J, ... of that
-// list.  So every XCD gets the same work whatever the routing (dealing whole
+// its routed range.  So every XCD gets the same work whatever the routing (dealing whole
 // (group, column tile) units round robin left the XCDs up to 2x apart with
 // skewed routing: T = 4096 down 144 -> 127 us, adversarial routing 400 ->
 // 358 us a layer), and a group stays on one XCD (two where a range ends
@@ -1001,14 +1044,14 @@ __device__ __forceinline__ void lds_tile(const GemmProblem& P, const TileRef& t,
 // cut into at most 8 runs).  Units are dealt round robin to the XCDs (routed
 // first, the shared ones numbered on).  An XCD's tiles are listed class by
 // class in decreasing estimated cost (class: problem and active blocks;
-// within a class, unit order), and its workgroup j walks tiles j, j + J, ...
-// of the list: the costly tiles start first and the second round is made of
-// the cheapest ones.  (The balanced placement made T = 512 131 -> 151 us: its
+// within a class, unit order): the costly tiles start first and the cheapest
+// ones fill the second round.  (The balanced placement made T = 512 131 -> 151 us: its
 // contiguous ranges put a range's costly tiles in one XCD's second round.)
 //
-// (A work queue -- atomic per-XCD counters, tiles taken as workgroups finish
-// them -- measured slower on this GPU: the counter round trips and their
-// broadcast cost more than the balance gained.)
+// A list's tiles are taken by ticket, the next one's round trip under the last
+// step of the tile before.  (Control words that share lines make this slow:
+// with the finished counts side by side and one count of all tiles taken, a
+// T = 64 layer took 107 us for 88.)
 //
 // Cost.  A tile's cost grows with its active 32-row blocks, and an int8
 // tile's more than a bf16 one's (the dequantisation is paid per tile).
@@ -1210,6 +1253,7 @@ __device__ __forceinline__ TileRef class_tile(const GemmProblem& P, const Units&
   t.pos0 = __builtin_amdgcn_readlane(hh ? q.start[1] : q.start[0], lane) + mt * BM;
   t.rows = min(BM, count - mt * BM);
   t.e = __builtin_amdgcn_readlane(hh ? q.e[1] : q.e[0], lane);
+  t.need = (count + BM - 1) / BM;
   return t;
 }
 
@@ -1264,23 +1308,111 @@ __device__ __forceinline__ Sched make_sched(const GemmProblem& a, const GemmProb
   return sd;
 }
 
-// The balanced placement's walk of the XCD's list.
+// A routed or shared tile by its active 32-row blocks.
 template <WKind W0, int NP>
-__device__ __forceinline__ void walk_balanced(const GemmProblem& a, const GemmProblem& b, char* lds_stages) {
+__device__ __forceinline__ int routed_tile(const GemmProblem& a, const TileRef& t, char* lds, const PhaseCtl& pc) {
+  constexpr int BMA = kLdsBM<W0>;
+  const int nact = (t.rows + 31) >> 5;
+  if constexpr (BMA == 128) {
+    if (nact == 4) return lds_tile<BMA, W0, NP, 4>(a, t, lds, pc);
+    if (nact == 3) return lds_tile<BMA, W0, NP, 3>(a, t, lds, pc);
+  } else {
+    static_assert(BMA == 64, "64- or 128-row tiles");
+  }
+  if (nact == 2) return lds_tile<BMA, W0, NP, 2>(a, t, lds, pc);
+  return lds_tile<BMA, W0, NP, 1>(a, t, lds, pc);
+}
+template <int NP>
+__device__ __forceinline__ int shared_tile(const GemmProblem& b, const TileRef& t, char* lds, const PhaseCtl& pc) {
+  constexpr int BMB = kLdsBM<kBf16KBlocked>;
+  static_assert(BMB == 64, "64-row shared tiles");
+  if (t.rows > 32) return lds_tile<BMB, kBf16KBlocked, NP, 2>(b, t, lds, pc);
+  return lds_tile<BMB, kBf16KBlocked, NP, 1>(b, t, lds, pc);
+}
+
+// The control words of a launch, zeroed before it, each on a line of its own
+// (agent-scope accesses skip the L2, and those of one line queue at the
+// memory): per phase (gate/up, down) and XCD a ticket counter and, after it,
+// the list's length + 1 once a workgroup has planned it; then the finished
+// gate/up tiles of each expert's rows and of each shared row tile.
+constexpr int kCtlDone = 2 * kXcds * kCtlLine;
+constexpr int kCtlSharedDep = 64;  // num_experts <= 64
+
+// Thread 0's value in every wave (the LDS word lies in the rings, idle between tiles).
+__device__ __forceinline__ int broadcast(int v, char* lds) {
+  if (threadIdx.x == 0) *(int*)lds = v;
+  lds_barrier();
+  v = __builtin_amdgcn_readfirstlane(*(const int*)lds);
+  lds_barrier();
+  return v;
+}
+
+// One phase of the launch (gate/up, NP = 2, or down, NP = 1) for a workgroup:
+// the tiles of its own XCD's list by ticket, then what is left of the others'.
+// So a workgroup goes on to the down tiles once every gate/up tile has been
+// taken by a running workgroup: a down tile's wait ends whatever else shares
+// the device.  plan(x) prepares XCD x's list and returns its length, run(it,
+// ctl) does tile `it` of it.  STEAL: take other lists' tiles at once, in both
+// phases (many tiles a list: T = 4096 363 -> 350 us).  Otherwise a list's few
+// remaining gate/up tiles are given kPatience polls (some microseconds) to be
+// taken by its own workgroups, which have it planned (taking them at once:
+// T = 291 92 -> 96 us, T = 64 87 -> 93).
+constexpr int kPatience = 16;
+template <int NP, bool STEAL, typename PlanFn, typename RunFn>
+__device__ __forceinline__ void walk(int32_t* ctl, char* lds, PlanFn&& plan, RunFn&& run) {
+  int32_t* lists = ctl + (NP == 2 ? 0 : kXcds) * kCtlLine;
+  const int own = (int)blockIdx.x % kXcds;
+  uint32_t unseen = (1u << kXcds) - 1;  // lists this workgroup has not run to their end
+  for (int x = own;;) {
+    const PhaseCtl pc{lists + x * kCtlLine, ctl + kCtlDone};
+    int v = 0;
+    if (threadIdx.x == 0) v = agent_add(pc.ticket, 1);
+    const int n = plan(x);
+    int it = broadcast(v, lds);
+    if (it == 0 && threadIdx.x == 0)
+      __hip_atomic_store(pc.ticket + 1, n + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    while (it < n) it = run(it, pc);
+    if (!STEAL && NP == 1) return;
+    unseen &= ~(1u << x);
+    if (threadIdx.x < kWave) {
+      // a bit per list whose tickets have not run past its length, or whose length is not known yet
+      const int32_t* p = lists + (int)threadIdx.x % kXcds * kCtlLine;
+      for (int k = 0;; ++k) {
+        const int taken = agent_load(p), len = agent_load(p + 1);
+        v = (int)((uint32_t)__ballot(len == 0 || taken < len - 1) & unseen);
+        if (STEAL || v == 0 || k == kPatience) break;
+        __builtin_amdgcn_s_sleep(8);
+      }
+    }
+    unseen = (uint32_t)broadcast(v, lds);
+    if (unseen == 0) return;
+    // the next list after the own one that may have tiles
+    x = (own + __builtin_ctz((unseen | (unseen << kXcds)) >> own)) % kXcds;
+  }
+}
+
+// The balanced placement's list of XCD x.  cols: gate/up column tiles of the
+// routed and the shared problem (a down tile waits for all of its rows').
+template <WKind W0, int NP>
+__device__ __forceinline__ void walk_balanced(const GemmProblem& a, const GemmProblem& b, int colsa, int colsb,
+                                              int32_t* ctl, char* lds_stages) {
   constexpr int bn = kWRowsWg / NP;
   constexpr int BMA = kLdsBM<W0>, BMB = kLdsBM<kBf16KBlocked>;
-  const int x = (int)blockIdx.x % kXcds;
-  const int j = (int)blockIdx.x / kXcds;
-  const int J = (int)gridDim.x / kXcds;
-  const Seq q = make_seq<BMA, BMB>(a, b, bn);
-  // the XCD's shared row tiles [b0, b1) and routed tiles [s0, s1)
+  Seq q;
+  bool made = false;
   const int rtb = (b.M + BMB - 1) / BMB;
-  const int b0 = rtb * x / kXcds, b1 = rtb * (x + 1) / kXcds;
-  const int nsh = (b1 - b0) * q.ntb;
-  const int s0 = seq_below<BMA>(a, q, (int64_t)q.ca * x / kXcds);
-  const int s1 = seq_below<BMA>(a, q, (int64_t)q.ca * (x + 1) / kXcds);
+  int b0 = 0, nsh = 0, s0 = 0;
+  // the XCD's shared row tiles [b0, b1) and routed tiles [s0, s1)
+  auto plan = [&](int x) __attribute__((always_inline)) {
+    if (!made) q = make_seq<BMA, BMB>(a, b, bn);
+    made = true;
+    b0 = rtb * x / kXcds;
+    nsh = (rtb * (x + 1) / kXcds - b0) * q.ntb;
+    s0 = seq_below<BMA>(a, q, (int64_t)q.ca * x / kXcds);
+    return nsh + seq_below<BMA>(a, q, (int64_t)q.ca * (x + 1) / kXcds) - s0;
+  };
   // tile i of the XCD's list: its problem, row tile and column tile
-  auto run = [&](int i) __attribute__((always_inline)) {
+  auto run = [&](int i, const PhaseCtl& pc) __attribute__((always_inline)) {
     if (i >= nsh) {
       i += s0 - nsh;
       // the last ranked group whose tiles start at or below i
@@ -1293,67 +1425,44 @@ __device__ __forceinline__ void walk_balanced(const GemmProblem& a, const GemmPr
       t.pos0 = __builtin_amdgcn_readlane(q.start, g) + mt * BMA;
       t.rows = min(BMA, count - mt * BMA);
       t.e = __builtin_amdgcn_readlane(q.e, g);
-      const int nact = (t.rows + 31) >> 5;
-      if constexpr (BMA == 128) {
-        if (nact == 4)
-          lds_tile<BMA, W0, NP, 4>(a, t, lds_stages);
-        else if (nact == 3)
-          lds_tile<BMA, W0, NP, 3>(a, t, lds_stages);
-        else if (nact == 2)
-          lds_tile<BMA, W0, NP, 2>(a, t, lds_stages);
-        else
-          lds_tile<BMA, W0, NP, 1>(a, t, lds_stages);
-      } else {
-        static_assert(BMA == 64, "64- or 128-row tiles");
-        if (nact == 2)
-          lds_tile<BMA, W0, NP, 2>(a, t, lds_stages);
-        else
-          lds_tile<BMA, W0, NP, 1>(a, t, lds_stages);
-      }
-    } else {
-      static_assert(BMB == 64, "64-row shared tiles");
-      const int mt = b0 + i / q.ntb;
-      const int cr = i - (mt - b0) * q.ntb;  // K range cr / ntr, column tile cr % ntr
-      const int ntr = q.ntb / parts_of(b);
-      TileRef t;
-      t.e = cr / ntr;
-      t.n0 = (cr - t.e * ntr) * bn;
-      t.pos0 = mt * BMB;
-      t.rows = min(BMB, b.M - mt * BMB);
-      if (t.rows > 32)
-        lds_tile<BMB, kBf16KBlocked, NP, 2>(b, t, lds_stages);
-      else
-        lds_tile<BMB, kBf16KBlocked, NP, 1>(b, t, lds_stages);
+      t.dep = t.e;
+      t.need = colsa * ((count + BMA - 1) / BMA);
+      return routed_tile<W0, NP>(a, t, lds_stages, pc);
     }
+    const int mt = b0 + i / q.ntb;
+    const int cr = i - (mt - b0) * q.ntb;  // K range cr / ntr, column tile cr % ntr
+    const int ntr = q.ntb / parts_of(b);
+    TileRef t;
+    t.e = cr / ntr;
+    t.n0 = (cr - t.e * ntr) * bn;
+    t.pos0 = mt * BMB;
+    t.rows = min(BMB, b.M - mt * BMB);
+    t.dep = kCtlSharedDep + mt;
+    t.need = colsb;
+    return shared_tile<NP>(b, t, lds_stages, pc);
   };
-  // Two rounds at most (small batches): the second round runs in reverse, so
-  // that the workgroups with the list's costliest first tiles take none and
-  // those with its cheapest take the rest.  More rounds walk in order.
-  const int n = nsh + s1 - s0;
-  const bool two = n <= 2 * J;
-  const int rounds = two ? 2 : (n - j + J - 1) / J;
-  for (int k = 0; k < rounds; ++k) {
-    const int it = two && k == 1 ? 2 * J - 1 - j : j + k * J;
-    if (it < n) run(it);
-  }
+  walk<NP, true>(ctl, lds_stages, plan, run);
 }
 
-// The by-class placement's walk of the XCD's list.
+// The by-class placement's list of XCD x.
 template <WKind W0, int NP>
-__device__ __forceinline__ void walk_classes(const GemmProblem& a, const GemmProblem& b, char* lds_stages) {
+__device__ __forceinline__ void walk_classes(const GemmProblem& a, const GemmProblem& b, int colsa, int colsb,
+                                             int32_t* ctl, char* lds_stages) {
   constexpr int bn = kWRowsWg / NP;
   constexpr int BMA = kLdsBM<W0>, BMB = kLdsBM<kBf16KBlocked>;
-  const int x = (int)blockIdx.x % kXcds;
   const int ntr = (b.N + bn - 1) / bn;  // the shared problem's column tiles, in every K range
   const int nta = (a.N + bn - 1) / bn, ntb = ntr * parts_of(b);
-  const int nga = a.rows.n_groups != nullptr ? ldc(a.rows.n_groups) : 1;
-  const int j = (int)blockIdx.x / kXcds;
-  const int J = (int)gridDim.x / kXcds;
-  const Units qa = plan_units<BMA>(a, nta, nga, x, 0);
-  const Units qb = plan_units<BMB>(b, ntb, 1, x, qa.n);  // dealt on from where the routed units ended
-  const Sched sd = make_sched<BMA, BMB>(a, b, qa, qb);
+  Units qa, qb;
+  Sched sd;
+  auto plan = [&](int x) __attribute__((always_inline)) {
+    const int nga = a.rows.n_groups != nullptr ? ldc(a.rows.n_groups) : 1;
+    qa = plan_units<BMA>(a, nta, nga, x, 0);
+    qb = plan_units<BMB>(b, ntb, 1, x, qa.n);  // dealt on from where the routed units ended
+    sd = make_sched<BMA, BMB>(a, b, qa, qb);
+    return sd.total;
+  };
   // tile `it` of the XCD's list: its class, then the class's tile
-  auto run = [&](int it) __attribute__((always_inline)) {
+  auto run = [&](int it, const PhaseCtl& pc) __attribute__((always_inline)) {
     int cls = sd.cls[0];
     bool found = false;
 #pragma unroll
@@ -1369,59 +1478,50 @@ __device__ __forceinline__ void walk_classes(const GemmProblem& a, const GemmPro
     }
     const int nact = cls & 255;
     if ((cls >> 8) == 0) {
-      if constexpr (BMA == 128) {
-        if (nact == 4)
-          lds_tile<BMA, W0, NP, 4>(a, class_tile<BMA>(a, qa, 4, it, bn), lds_stages);
-        else if (nact == 3)
-          lds_tile<BMA, W0, NP, 3>(a, class_tile<BMA>(a, qa, 3, it, bn), lds_stages);
-        else if (nact == 2)
-          lds_tile<BMA, W0, NP, 2>(a, class_tile<BMA>(a, qa, 2, it, bn), lds_stages);
-        else
-          lds_tile<BMA, W0, NP, 1>(a, class_tile<BMA>(a, qa, 1, it, bn), lds_stages);
-      } else {
-        static_assert(BMA == 64, "64- or 128-row tiles");
-        if (nact == 2)
-          lds_tile<BMA, W0, NP, 2>(a, class_tile<BMA>(a, qa, 2, it, bn), lds_stages);
-        else
-          lds_tile<BMA, W0, NP, 1>(a, class_tile<BMA>(a, qa, 1, it, bn), lds_stages);
-      }
-    } else {
-      static_assert(BMB == 64, "64-row shared tiles");
-      TileRef t = class_tile<BMB>(b, qb, nact, it, bn);
-      const int cr = t.n0 / bn;  // K range cr / ntr, column tile cr % ntr
-      t.e = cr / ntr;
-      t.n0 = (cr - t.e * ntr) * bn;
-      if (nact == 2)
-        lds_tile<BMB, kBf16KBlocked, NP, 2>(b, t, lds_stages);
-      else
-        lds_tile<BMB, kBf16KBlocked, NP, 1>(b, t, lds_stages);
+      TileRef t = class_tile<BMA>(a, qa, nact, it, bn);
+      t.dep = t.e;
+      t.need *= colsa;
+      return routed_tile<W0, NP>(a, t, lds_stages, pc);
     }
+    TileRef t = class_tile<BMB>(b, qb, nact, it, bn);
+    const int cr = t.n0 / bn;  // K range cr / ntr, column tile cr % ntr
+    t.e = cr / ntr;
+    t.n0 = (cr - t.e * ntr) * bn;
+    t.dep = kCtlSharedDep + t.pos0 / BMB;
+    t.need = colsb;
+    return shared_tile<NP>(b, t, lds_stages, pc);
   };
-  // Two rounds at most (small batches): the second round runs in reverse, so
-  // that the workgroups with the costliest first tiles take the cheapest
-  // second ones (at T = 512, gate/up 70 -> 66 us).  More rounds walk in
-  // order (reversing every other round made T = 4096 slower).
-  const bool two = sd.total <= 2 * J;
-  const int rounds = two ? 2 : (sd.total - j + J - 1) / J;
-  for (int k = 0; k < rounds; ++k) {
-    const int it = two && k == 1 ? 2 * J - 1 - j : j + k * J;
-    if (it < sd.total) run(it);
+  walk<NP, false>(ctl, lds_stages, plan, run);
+}
+
+// Gate/up (a, b) and down (c, d) of the routed and the shared experts in one
+// persistent launch.  A workgroup that has no gate/up tile left goes on to the
+// down tiles, each of which waits for its own expert's (or shared row tile's)
+// gate/up tiles; with a launch per phase, every workgroup waited for the last
+// gate/up tile, and the second launch planned and filled its pipelines again.
+// h crosses XCDs inside the launch: stored past the L2, then counted, and
+// loaded past the L2 (which costs nothing here: each row tile's few readers).
+// Measured (a layer, two launches -> one): int8 T = 291 105 -> 94 us, T = 512
+// 112 -> 109, T = 4096 371 -> 349, bf16 T = 1531 250 -> 224.
+template <WKind W0, bool BAL>
+__global__ void __launch_bounds__(kGThreads, kWgPerCu) k_moe_layer(GemmProblem a, GemmProblem b, GemmProblem c,
+                                                                   GemmProblem d, int32_t* ctl) {
+  extern __shared__ __attribute__((aligned(16))) char lds_stages[];
+  constexpr int bn = kWRowsWg / 2;
+  const int colsa = (a.N + bn - 1) / bn, colsb = (b.N + bn - 1) / bn;
+  if constexpr (BAL) {
+    walk_balanced<W0, 2>(a, b, colsa, colsb, ctl, lds_stages);
+    walk_balanced<W0, 1>(c, d, colsa, colsb, ctl, lds_stages);
+  } else {
+    walk_classes<W0, 2>(a, b, colsa, colsb, ctl, lds_stages);
+    walk_classes<W0, 1>(c, d, colsa, colsb, ctl, lds_stages);
   }
 }
 
-template <WKind W0, int NP, bool BAL>
-__global__ void __launch_bounds__(kGThreads, kWgPerCu) k_moe_gemm_lds(GemmProblem a, GemmProblem b) {
-  extern __shared__ __attribute__((aligned(16))) char lds_stages[];
-  if constexpr (BAL)
-    walk_balanced<W0, NP>(a, b, lds_stages);
-  else
-    walk_classes<W0, NP>(a, b, lds_stages);
-}
-
-// Workgroups of the LDS-staged grid: every CU's resident share, a whole
-// number per XCD (the same for both placements).
-template <WKind W0, int NP>
-hipError_t moe_gemm_lds_grid(int* grid) {
+// Workgroups of the layer's grid: every CU's resident share, a whole number
+// per XCD (the same for both placements).
+template <WKind W0>
+hipError_t moe_layer_grid(int* grid) {
   constexpr size_t lds = kLdsBytes<W0>;
   static std::atomic<int> cached{0};
   int g = cached.load(std::memory_order_relaxed);
@@ -1429,10 +1529,10 @@ hipError_t moe_gemm_lds_grid(int* grid) {
     int dev = 0, cus = 0, per_cu = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    for (const void* f : {(const void*)k_moe_gemm_lds<W0, NP, false>, (const void*)k_moe_gemm_lds<W0, NP, true>})
+    for (const void* f : {(const void*)k_moe_layer<W0, false>, (const void*)k_moe_layer<W0, true>})
       if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e == hipSuccess)
-      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_moe_gemm_lds<W0, NP, false>, kGThreads, lds);
+      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_moe_layer<W0, false>, kGThreads, lds);
     if (e != hipSuccess) return e;
     g = (cus / kXcds > 0 ? cus / kXcds : 1) * (per_cu > 0 ? per_cu : 1) * kXcds;
     cached.store(g, std::memory_order_relaxed);
@@ -1441,23 +1541,30 @@ hipError_t moe_gemm_lds_grid(int* grid) {
   return hipSuccess;
 }
 
-// The balanced placement once the launch's tiles (bounded from the rows)
-// exceed two rounds of the grid.
-template <WKind W0, int NP>
-hipError_t launch_moe_gemm_lds(const GemmProblem& routed, const GemmProblem& shared, hipStream_t s,
-                               const char* name) {
+// Tiles of a phase, bounded from the rows.
+template <WKind W0>
+int64_t tile_bound(const GemmProblem& routed, const GemmProblem& shared, int shared_parts) {
+  const int bn = kWRowsWg / (routed.swiglu ? 2 : 1);
+  constexpr int BMA = kLdsBM<W0>, BMB = kLdsBM<kBf16KBlocked>;
+  return (int64_t)((routed.N + bn - 1) / bn) * ((routed.M + BMA - 1) / BMA + routed.max_groups) +
+         (int64_t)((shared.N + bn - 1) / bn) * shared_parts * ((shared.M + BMB - 1) / BMB);
+}
+
+// The balanced placement once the tiles of a phase exceed two rounds of the
+// grid (the by-class plan holds kMaxUnits units of a problem; the gate/up
+// phase is the larger one where ffn is near hidden).
+template <WKind W0>
+hipError_t launch_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn, const GemmProblem& sdn,
+                        int32_t* ctl, hipStream_t s) {
   constexpr size_t lds = kLdsBytes<W0>;
   int grid = 0;
-  const hipError_t e = moe_gemm_lds_grid<W0, NP>(&grid);
+  const hipError_t e = moe_layer_grid<W0>(&grid);
   if (e != hipSuccess) return e;
-  constexpr int bn = kWRowsWg / NP;
-  constexpr int BMA = kLdsBM<W0>, BMB = kLdsBM<kBf16KBlocked>;
-  const int64_t tiles = (int64_t)((routed.N + bn - 1) / bn) * ((routed.M + BMA - 1) / BMA + routed.max_groups) +
-                        (int64_t)((shared.N + bn - 1) / bn) * parts_of(shared) * ((shared.M + BMB - 1) / BMB);
-  if (tiles > 2 * (int64_t)grid)
-    UOCR_LAUNCH(name, (k_moe_gemm_lds<W0, NP, true>), dim3(grid), dim3(kGThreads), lds, s, routed, shared);
+  const int64_t rounds2 = std::min(2 * (int64_t)grid, (int64_t)kMaxUnits);
+  if (tile_bound<W0>(gu, sgu, 1) > rounds2 || tile_bound<W0>(dn, sdn, parts_of(sdn)) > rounds2)
+    UOCR_LAUNCH("gemm_layer", (k_moe_layer<W0, true>), dim3(grid), dim3(kGThreads), lds, s, gu, sgu, dn, sdn, ctl);
   else
-    UOCR_LAUNCH(name, (k_moe_gemm_lds<W0, NP, false>), dim3(grid), dim3(kGThreads), lds, s, routed, shared);
+    UOCR_LAUNCH("gemm_layer", (k_moe_layer<W0, false>), dim3(grid), dim3(kGThreads), lds, s, gu, sgu, dn, sdn, ctl);
   return hipGetLastError();
 }
 
@@ -1495,48 +1602,50 @@ int gemm_shared_parts(const GemmProblem& routed, const GemmProblem& shared) {
   if (shared.kind != kBf16KBlocked || shared.swiglu || shared.K % (2 * 2 * BK)) return 1;
   int grid = 0;
   const bool int8 = routed.kind == kInt8Rows;
-  const hipError_t e = routed.swiglu ? (int8 ? moe_gemm_lds_grid<kInt8Rows, 2>(&grid) : moe_gemm_lds_grid<kBf16Rows, 2>(&grid))
-                                     : (int8 ? moe_gemm_lds_grid<kInt8Rows, 1>(&grid) : moe_gemm_lds_grid<kBf16Rows, 1>(&grid));
+  const hipError_t e = int8 ? moe_layer_grid<kInt8Rows>(&grid) : moe_layer_grid<kBf16Rows>(&grid);
   if (e != hipSuccess || grid <= 0) return 1;
-  const int bn = kWRowsWg / (routed.swiglu ? 2 : 1);
-  const int BMA = int8 ? kLdsBM<kInt8Rows> : kLdsBM<kBf16Rows>, BMB = kLdsBM<kBf16KBlocked>;
-  const int64_t tiles = (int64_t)((routed.N + bn - 1) / bn) * ((routed.M + BMA - 1) / BMA + routed.max_groups) +
-                        (int64_t)((shared.N + bn - 1) / bn) * 2 * ((shared.M + BMB - 1) / BMB);
+  const int64_t tiles = int8 ? tile_bound<kInt8Rows>(routed, shared, 2) : tile_bound<kBf16Rows>(routed, shared, 2);
   return tiles <= 2 * (int64_t)grid ? 2 : 1;
 }
 
-hipError_t launch_gemm_pair(const GemmProblem& routed, const GemmProblem& shared, int bm, hipStream_t s, bool vec) {
-  const bool gu = routed.swiglu != 0;
-  const char* name = gu ? "gemm_gateup" : "gemm_down";
-  if (routed.N % 32 || shared.N % 32 || routed.K % (2 * BK) || shared.K % (2 * BK)) return hipErrorInvalidValue;
+static bool gemm_shapes_ok(const GemmProblem& routed, const GemmProblem& shared) {
+  if (routed.N % 32 || shared.N % 32 || routed.K % (2 * BK) || shared.K % (2 * BK)) return false;
   // K ranges: the shared problem only, each an even number of K steps, fp32 sums
   if (parts_of(shared) > 1 && (shared.K % (parts_of(shared) * 2 * BK) || shared.swiglu || shared.outf == nullptr))
-    return hipErrorInvalidValue;
-  if (routed.kind == kInt8Rows && (routed.K % routed.groups || (routed.K / routed.groups) % BK))
-    return hipErrorInvalidValue;
-  if ((routed.kind == kInt8Rows && routed.groups > kMaxScaleGroups) || routed.max_groups > kWave) {
-    // groups finer than K / 16 (the fragment-load kernel reads each step's scale itself), or more
-    // routed groups than the LDS-staged kernel's placement holds (one a lane)
-    if (routed.kind == kInt8Rows)
-      return gu ? launch_moe_gemm<64, kInt8Rows, 2, false>(routed, shared, s, name)
-                : launch_moe_gemm<64, kInt8Rows, 1, false>(routed, shared, s, name);
-    return gu ? launch_moe_gemm<64, kBf16Rows, 2, false>(routed, shared, s, name)
-              : launch_moe_gemm<64, kBf16Rows, 1, false>(routed, shared, s, name);
-  }
-  if (!vec) {  // weights at any alignment: 64-row tiles only
-    if (bm != 64) return hipErrorInvalidValue;
-    if (routed.kind == kInt8Rows)
-      return gu ? launch_moe_gemm<64, kInt8Rows, 2, false>(routed, shared, s, name)
-                : launch_moe_gemm<64, kInt8Rows, 1, false>(routed, shared, s, name);
-    return gu ? launch_moe_gemm<64, kBf16Rows, 2, false>(routed, shared, s, name)
-              : launch_moe_gemm<64, kBf16Rows, 1, false>(routed, shared, s, name);
-  }
-  // 16-byte aligned operands: the LDS-staged kernel (its tile heights are its own)
+    return false;
+  return routed.kind != kInt8Rows || (routed.K % routed.groups == 0 && (routed.K / routed.groups) % BK == 0);
+}
+
+int moe_layer_ctl_words(int64_t tokens) {
+  return kCtlDone +
+         kCtlLine * (kCtlSharedDep + (int)((tokens + kLdsBM<kBf16KBlocked> - 1) / kLdsBM<kBf16KBlocked>));
+}
+
+// 16-byte aligned weights, at most kMaxScaleGroups int8 groups a row, and a
+// lane per routed group in the placement's plan; the fragment-load kernel
+// takes the rest, a launch per phase.
+bool moe_layer_ok(const GemmProblem& gu, const GemmProblem& dn, bool vec) {
+  if (!vec || gu.max_groups > kWave) return false;
+  return gu.kind != kInt8Rows || (gu.groups <= kMaxScaleGroups && dn.groups <= kMaxScaleGroups);
+}
+
+hipError_t launch_moe_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn,
+                            const GemmProblem& sdn, int32_t* ctl, hipStream_t s) {
+  if (!gemm_shapes_ok(gu, sgu) || !gemm_shapes_ok(dn, sdn)) return hipErrorInvalidValue;
+  return gu.kind == kInt8Rows ? launch_layer<kInt8Rows>(gu, sgu, dn, sdn, ctl, s)
+                              : launch_layer<kBf16Rows>(gu, sgu, dn, sdn, ctl, s);
+}
+
+// One phase of the layer with the fragment-load kernel (64-row tiles).
+hipError_t launch_gemm_pair(const GemmProblem& routed, const GemmProblem& shared, hipStream_t s) {
+  const bool gu = routed.swiglu != 0;
+  const char* name = gu ? "gemm_gateup" : "gemm_down";
+  if (!gemm_shapes_ok(routed, shared)) return hipErrorInvalidValue;
   if (routed.kind == kInt8Rows)
-    return gu ? launch_moe_gemm_lds<kInt8Rows, 2>(routed, shared, s, name)
-              : launch_moe_gemm_lds<kInt8Rows, 1>(routed, shared, s, name);
-  return gu ? launch_moe_gemm_lds<kBf16Rows, 2>(routed, shared, s, name)
-            : launch_moe_gemm_lds<kBf16Rows, 1>(routed, shared, s, name);
+    return gu ? launch_moe_gemm<64, kInt8Rows, 2, false>(routed, shared, s, name)
+              : launch_moe_gemm<64, kInt8Rows, 1, false>(routed, shared, s, name);
+  return gu ? launch_moe_gemm<64, kBf16Rows, 2, false>(routed, shared, s, name)
+            : launch_moe_gemm<64, kBf16Rows, 1, false>(routed, shared, s, name);
 }
 
 }  // namespace uocr

@@ -732,6 +732,8 @@ __global__ void __launch_bounds__(256) k_group_scatter_hist(const int32_t* __res
   const int tid = (int)threadIdx.x;
   const int e = tid & 63;
   const int c = tid >> 6;
+  if (b == 0 && g.ctl != nullptr)
+    for (int i = tid; i < g.nctl; i += 256) stg(g.ctl + i, 0);
   // four threads per expert, each over every fourth counting workgroup, 16
   // loads in flight at a time (indices past the last block re-read it and
   // are not counted)

@@ -115,6 +115,8 @@ struct GroupTables {
   int32_t* group_rows;    // [R]
   int32_t* tile_start;    // [E + 1] prefix of ceil(count / bm), may be null
   int32_t* inv;           // [R] position of row r in group_rows, may be null
+  int32_t* ctl;           // [nctl] words the prefill grouping clears for a later kernel, may be null
+  int nctl;
 };
 // Groups R rows by their clamped expert id (ascending expert).
 hipError_t launch_group(const int32_t* ids, int R, int E, int bm, const GroupTables& g, hipStream_t s);
@@ -181,12 +183,18 @@ struct GemmProblem {
   int kparts;
   int64_t part_stride;
 };
-// bm: rows per tile, 64 or 128.  vec: every weight pointer is 16-byte
-// aligned; else the weights are read at any alignment (bm must be 64), with
-// the same bits.  N must be a multiple of 32 and K of 128 (and of the int8
-// group, itself a multiple of 64); a routed problem has at most 64 groups.
-hipError_t launch_gemm_pair(const GemmProblem& routed, const GemmProblem& shared, int bm, hipStream_t s,
-                            bool vec = true);
+// N must be a multiple of 32 and K of 128 (and of the int8 group, itself a
+// multiple of 64); a routed problem has at most 64 groups.
+//
+// Gate/up and down of a layer in one launch: dn and sdn read what gu and sgu
+// write.  ctl: moe_layer_ctl_words(tokens) words, zero before the launch (the
+// grouping's launch clears them).  moe_layer_ok: what it takes.
+int moe_layer_ctl_words(int64_t tokens);
+bool moe_layer_ok(const GemmProblem& gu, const GemmProblem& dn, bool vec);
+hipError_t launch_moe_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn,
+                            const GemmProblem& sdn, int32_t* ctl, hipStream_t s);
+// One phase, weights at any alignment, with the same bits.
+hipError_t launch_gemm_pair(const GemmProblem& routed, const GemmProblem& shared, hipStream_t s);
 // The K ranges to cut the shared problem into for this pair (1 or 2).
 int gemm_shared_parts(const GemmProblem& routed, const GemmProblem& shared);
 

@@ -936,6 +936,8 @@ static PrefillBufs carve_prefill(Carve& c, const uocr_moe_layer* L, int64_t T) {
   d.sh = c.take<float>(2 * T * L->hidden);  // the shared experts' down sums, in up to two K ranges
   // (the T < 2048 routing's 4-token blocks outnumber the T >= 2048 one's 16-token blocks)
   d.hist = c.take<int32_t>((int64_t)fused_route_blocks((int)T) * L->num_experts);
+  d.g.nctl = moe_layer_ctl_words(T);
+  d.g.ctl = c.take<int32_t>(d.g.nctl);
   return d;
 }
 
@@ -1343,9 +1345,6 @@ int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden, co
   sgu.swiglu = 1;
   sgu.outb = d.hsb;
   sgu.ldo = Fs;
-  e = launch_gemm_pair(gu, sgu, BM, s, vec);
-  if (e != hipSuccess) return hip_fail(err, errlen, op, e);
-
   GemmProblem dn = gu;
   dn.a = d.hb;
   dn.lda = F;
@@ -1378,7 +1377,12 @@ int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden, co
   // launch's longest at T = 512 (down 43 -> 35 us).
   sdn.kparts = gemm_shared_parts(dn, sdn);
   sdn.part_stride = T * H;
-  e = launch_gemm_pair(dn, sdn, BM, s, vec);
+  if (moe_layer_ok(gu, dn, vec && aligned16(ws))) {
+    e = launch_moe_layer(gu, sgu, dn, sdn, d.g.ctl, s);
+  } else {
+    e = launch_gemm_pair(gu, sgu, s);
+    if (e == hipSuccess) e = launch_gemm_pair(dn, sdn, s);
+  }
   if (e == hipSuccess)
     e = launch_combine(out, d.y, H, d.wts, d.g.inv, d.sh, (int)T, H, (int)L->top_k, s, sdn.kparts);
   if (e == hipSuccess && expert_ids) e = hipMemcpyAsync(expert_ids, d.ids, R * sizeof(int32_t), hipMemcpyDeviceToDevice, s);
