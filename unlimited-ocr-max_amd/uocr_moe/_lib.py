@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 from pathlib import Path
 
 import torch  # noqa: F401  (loads the HIP runtime the library links against)
@@ -79,6 +80,16 @@ _RESTYPES = {"uocr_moe_workspace_bytes": _sz, "uocr_paged_attention_workspace_by
 _LIB: ctypes.CDLL | None = None
 
 
+class _Err(threading.local):
+    """Each thread's error message buffer (empty between calls)."""
+
+    def __init__(self) -> None:
+        self.buffer = ctypes.create_string_buffer(ERRLEN)
+
+
+_ERR = _Err()
+
+
 def load() -> ctypes.CDLL:
     """The library with its signatures declared; raises if it was not built."""
     global _LIB
@@ -99,10 +110,12 @@ def load() -> ctypes.CDLL:
 
 def call(name: str, *args) -> None:
     """Calls an entry point that takes a trailing ``(err, errlen)`` and raises its message on failure."""
-    err = ctypes.create_string_buffer(ERRLEN)
-    rc = getattr(load(), name)(*args, err, ERRLEN)
+    err = _ERR.buffer
+    rc = getattr(_LIB or load(), name)(*args, err, ERRLEN)
     if rc != 0:
-        raise UocrError(err.value.decode() or f"{name} failed with code {rc}")
+        message = err.value.decode()
+        err.value = b""
+        raise UocrError(message or f"{name} failed with code {rc}")
 
 
 def timing_begin(capacity: int) -> None:

@@ -43,7 +43,8 @@ DENSE_MIN_ITEMS = 2048
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The raw handle of torch's current stream on ``t``'s device (a Stream object for it costs a microsecond)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _gpu(op: str, name: str, t: torch.Tensor, dtype: torch.dtype, rank: int) -> torch.Tensor:
@@ -53,9 +54,9 @@ def _gpu(op: str, name: str, t: torch.Tensor, dtype: torch.dtype, rank: int) -> 
         raise TypeError(f"{op}: {name} must be {dtype}, got {t.dtype}")
     if t.dim() != rank:
         raise ValueError(f"{op}: {name} must be rank {rank}, got shape {tuple(t.shape)}")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{op}: {name} must be on the GPU, got {t.device}")
-    return t.contiguous()
+    return t if t.is_contiguous() else t.contiguous()
 
 
 def _out(op: str, name: str, t: torch.Tensor, dtype: torch.dtype, rank: int) -> torch.Tensor:
@@ -145,13 +146,15 @@ def dense_bf16_qmv(x, w, *, tile: int | None = None, out: torch.Tensor | None = 
     op = "dense_bf16_qmv"
     x = _gpu(op, "x", x, torch.float32, 2)
     w = _gpu(op, "w", w, torch.bfloat16, 3)
+    (rows, kdim), (blocks, n, kblock) = x.shape, w.shape
     if tile is None:
-        tile = _rows_per_read(int(x.shape[0]), int(w.shape[1]))
+        tile = _rows_per_read(rows, n)
     if out is None:
-        out = torch.empty((x.shape[0], w.shape[1]), dtype=torch.float32, device=x.device)
-    out = _out(op, "result", out, torch.float32, 2)
-    _lib.call("uocr_dense_bf16_qmv", out.data_ptr(), out.shape[0], out.shape[1], x.data_ptr(), x.shape[0], x.shape[1],
-              w.data_ptr(), *w.shape, int(tile), _stream(x))
+        out = x.new_empty((rows, n))
+    else:
+        out = _out(op, "result", out, torch.float32, 2)
+    _lib.call("uocr_dense_bf16_qmv", out.data_ptr(), *out.shape, x.data_ptr(), rows, kdim, w.data_ptr(), blocks, n,
+              kblock, int(tile), _stream(x))
     return out
 
 
@@ -385,7 +388,7 @@ def paged_decode_attention_qkv(qkv, positions, cos_table, sin_table, *, heads: i
     bits: ``qkv [B, 3 * heads * head_dim]`` (q, k, v side by side, q and k before RoPE; rows may be
     strided) is one fused projection's output (unlimited_ocr_max/decoder.py:487-492 with :425-437)."""
     op = "paged_decode_attention_qkv"
-    if not isinstance(qkv, torch.Tensor) or qkv.dtype != torch.float32 or qkv.dim() != 2 or qkv.device.type != "cuda":
+    if not isinstance(qkv, torch.Tensor) or qkv.dtype != torch.float32 or qkv.dim() != 2 or not qkv.is_cuda:
         raise ValueError(f"{op}: qkv must be an fp32 [rows, 3 * heads * head_dim] GPU tensor")
     if qkv.stride(1) != 1:
         qkv = qkv.contiguous()
@@ -400,7 +403,7 @@ def paged_decode_attention_qkv(qkv, positions, cos_table, sin_table, *, heads: i
         raise ValueError(f"{op}: positions or the cos/sin tables do not fit {rows} rows")
     blocks = kv.kv_blocks
     if not isinstance(blocks, torch.Tensor) or blocks.dtype != torch.float32 or blocks.dim() != 6 or \
-            blocks.device.type != "cuda" or not blocks.is_contiguous():
+            not blocks.is_cuda or not blocks.is_contiguous():
         raise ValueError(f"{op}: kv_blocks must be a contiguous f32 [pages, 2, layers, page_size, heads, head_dim]")
     pages, two, layers, page_size, bh, bd = blocks.shape
     if two != 2 or (bh, bd) != (heads, head_dim):
@@ -411,8 +414,9 @@ def paged_decode_attention_qkv(qkv, positions, cos_table, sin_table, *, heads: i
     if lookup.shape[0] != rows or attend.shape[0] != rows or write.shape[0] != rows:
         raise ValueError(f"{op}: the step metadata is not for {rows} rows")
     if out is None:
-        out = torch.empty((rows, heads, head_dim), device=qkv.device, dtype=torch.float32)
-    out = _out(op, "out", out, torch.float32, 3)
+        out = qkv.new_empty((rows, heads, head_dim))
+    else:
+        out = _out(op, "out", out, torch.float32, 3)
     ws, ws_bytes = (None, 0) if workspace is None else (workspace.data_ptr(), workspace.numel() * workspace.element_size())
     _lib.call("uocr_paged_decode_attention_qkv", out.data_ptr(), qkv.data_ptr(), rows, heads, head_dim, qkv.stride(0),
               positions.data_ptr(), cos_table.data_ptr(), sin_table.data_ptr(), cos_table.shape[0],
