@@ -70,14 +70,19 @@ __device__ __forceinline__ void rope_pair(float& lo, float& hi, const float* c, 
   lo = l * ldg(c + d) - h * ldg(s + d);
   hi = h * ldg(c + d + kD / 2) + l * ldg(s + d + kD / 2);
 }
-__device__ __forceinline__ void rope_pair4(f32x4& lo, f32x4& hi, const float* c, const float* s, int d) {
+// Four pairs, their cos and sin elements given.
+__device__ __forceinline__ void rope_pair4(f32x4& lo, f32x4& hi, f32x4 cl, f32x4 ch, f32x4 sl, f32x4 sh) {
+#pragma clang fp contract(off)
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    float l = lo[e], h = hi[e];
-    rope_pair(l, h, c, s, d + e);
-    lo[e] = l;
-    hi[e] = h;
+    const float l = lo[e], h = hi[e];
+    lo[e] = l * cl[e] - h * sl[e];
+    hi[e] = h * ch[e] + l * sh[e];
   }
+}
+// Four floats of a table row (4-byte aligned).
+__device__ __forceinline__ f32x4 load4(const float* p) {
+  return f32x4{ldg(p), ldg(p + 1), ldg(p + 2), ldg(p + 3)};
 }
 // Element d of the rotated row x.
 __device__ __forceinline__ float rope_elem(const float* x, const float* c, const float* s, int d) {
@@ -91,12 +96,6 @@ __device__ __forceinline__ float* row_ptr(const PagedArgs& a, int b, int h, int 
   const uint32_t page = min(ldg(a.lookup + (int64_t)b * a.lookup_cols + r / a.P), (uint32_t)(a.pages - 1));
   return a.pool + (int64_t)page * a.page_stride + kv * a.kv_stride + a.layer_off +
          (int64_t)(r % a.P) * a.slot_stride + (int64_t)h * kD;
-}
-
-// Row r0 of a split (its rows share one page: the page size is a multiple of
-// the split): the k (kv = 0) or v values, rows slot_stride floats apart.
-__device__ __forceinline__ const float* split_base(const PagedArgs& a, int b, int h, int r0, int kv) {
-  return row_ptr(a, b, h, r0, kv);
 }
 
 // Partials cross workgroups (and XCDs, whose L2s are not coherent with one
@@ -150,51 +149,70 @@ __device__ __forceinline__ float combine_splits(const float* p, int splits, int 
 // max and sum of exp into dst, or, given `direct`, the normalised output there.
 __device__ __forceinline__ void split_partial(const PagedArgs& a, const float* __restrict__ q,
                                               const float* __restrict__ k_new, const float* __restrict__ v_new,
-                                              float scale, int w_idx, int64_t bh, int b, int h, int r0, int r1,
-                                              float* sc, float* red, f32x4 (*vsum)[kD / 4], float* direct,
-                                              float* dst) {
+                                              float scale, int w_idx, int pos, int b, int h, int r0, int r1,
+                                              const float* kbase, const float* vbase, float* sc, float* red,
+                                              f32x4 (*vsum)[kD / 4], float* direct, float* dst) {
   const int tid = (int)threadIdx.x;
   // ---- every load of the split first: k (8 lanes per row, a load instruction covering 128 contiguous
-  // bytes of a row) and v (32 lanes per row, a float4 each).  Rows past the attended ones are still in
-  // the split's page (the page size is a multiple of the split), so the loads need no guard; their
-  // values are masked below.
+  // bytes of a row) and v (32 lanes per row, a float4 each).  Lanes past the attended rows repeat the
+  // last one's loads (no branch, and no bytes of rows that are not attended); their values are masked
+  // below.  The step's metadata, the pool row's address and q's tables come before and cost one round
+  // trip each, under no other load (8 rows of up to 640 / 1200: 13.4 -> 12.9, 23.5 -> 22.4 us, of which
+  // the bytes are 7 and 14).
   const int n = r1 - r0;
   const int sub = tid % kLanesPerRow, rg = tid / kLanesPerRow;
   const int c = tid % (kD / 4), g = tid / (kD / 4);
   const int64_t qoff = (int64_t)b * a.in_stride + (int64_t)h * kD;  // row b, head h of q / k_new / v_new
   const float* qh = q + qoff + sub * 4;
-  const float* rc = nullptr;
-  const float* rs = nullptr;
-  if (a.positions != nullptr) {
-    const int pos = min(max(ldg(a.positions + b), 0), a.table_rows - 1);  // device data: clamped into the table
-    rc = a.cos_t + (int64_t)pos * kD;
-    rs = a.sin_t + (int64_t)pos * kD;
-  }
-  const float* kbase = split_base(a, b, h, r0, 0);
-  const float* vbase = split_base(a, b, h, r0, 1);
+  const float* rc = a.positions != nullptr ? a.cos_t + (int64_t)pos * kD : nullptr;
+  const float* rs = a.positions != nullptr ? a.sin_t + (int64_t)pos * kD : nullptr;
   f32x4 qv[4], kv[kKRows][4], vv[kVRows];
+  f32x4 cv[4], sv[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) qv[u] = *(const UOCR_GLOBAL f32x4*)(qh + 32 * u);
-  if (rc != nullptr) {  // lane elements d = sub*4 + 32u + e: u = 0, 1 pair with u = 2, 3
-    rope_pair4(qv[0], qv[2], rc, rs, sub * 4);
-    rope_pair4(qv[1], qv[3], rc, rs, 32 + sub * 4);
+  if (rc != nullptr) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      cv[u] = load4(rc + sub * 4 + 32 * u);
+      sv[u] = load4(rs + sub * 4 + 32 * u);
+    }
   }
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int j = 0; j < kKRows; ++j) {
-    const int i = rg + j * kRowsPerPass;
+    const int i = min(rg + j * kRowsPerPass, n - 1);
     const float* kr = (r0 + i == w_idx ? k_new + qoff : kbase + (int64_t)i * a.slot_stride) + sub * 4;
 #pragma unroll
     for (int u = 0; u < 4; ++u) kv[j][u] = *(const UOCR_GLOBAL f32x4*)(kr + 32 * u);
-    if (rc != nullptr && r0 + i == w_idx) {  // the new row, read unrotated
-      rope_pair4(kv[j][0], kv[j][2], rc, rs, sub * 4);
-      rope_pair4(kv[j][1], kv[j][3], rc, rs, 32 + sub * 4);
-    }
   }
+  __builtin_amdgcn_sched_barrier(0);
+  // q is rotated while the keys are on their way (its own loads came first), which frees the registers that
+  // the values' loads take
+  if (rc != nullptr) {  // lane elements d = sub*4 + 32u + e: u = 0, 1 pair with u = 2, 3
+    rope_pair4(qv[0], qv[2], cv[0], cv[2], sv[0], sv[2]);
+    rope_pair4(qv[1], qv[3], cv[1], cv[3], sv[1], sv[3]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int j = 0; j < kVRows; ++j) {
-    const int i = g + j * kValueGroups;
+    const int i = min(g + j * kValueGroups, n - 1);
     const float* vr = r0 + i == w_idx ? v_new + qoff : vbase + (int64_t)i * a.slot_stride;
     vv[j] = *(const UOCR_GLOBAL f32x4*)(vr + 4 * c);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (rc != nullptr) {
+#pragma unroll
+    for (int j = 0; j < kKRows; ++j) {
+      if (r0 + min(rg + j * kRowsPerPass, n - 1) == w_idx) {  // the new row, read unrotated
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          cv[u] = load4(rc + sub * 4 + 32 * u);
+          sv[u] = load4(rs + sub * 4 + 32 * u);
+        }
+        rope_pair4(kv[j][0], kv[j][2], cv[0], cv[2], sv[0], sv[2]);
+        rope_pair4(kv[j][1], kv[j][3], cv[1], cv[3], sv[1], sv[3]);
+      }
+    }
   }
   // ---- scores
 #pragma unroll
@@ -274,7 +292,7 @@ __device__ __forceinline__ void split_partial(const PagedArgs& a, const float* _
 // splits - 1 returns splits - 1 to exactly one workgroup and leaves the counter
 // at 0 again.  Without counters the partials wait for k_attn_combine.  One
 // split writes the output directly.
-__global__ void __launch_bounds__(kThreads) k_attn_partial(PagedArgs a, const float* __restrict__ q,
+__global__ void __launch_bounds__(kThreads, 4) k_attn_partial(PagedArgs a, const float* __restrict__ q,
                                                            const float* __restrict__ k_new,
                                                            const float* __restrict__ v_new, float scale,
                                                            float* __restrict__ part, int splits,
@@ -283,31 +301,20 @@ __global__ void __launch_bounds__(kThreads) k_attn_partial(PagedArgs a, const fl
   __shared__ float red[kThreads / 64];
   __shared__ f32x4 vsum[kValueGroups - 1][kD / 4];
   __shared__ uint32_t last;
-  const int s = (int)blockIdx.x, h = (int)blockIdx.y, b = (int)blockIdx.z;
+  const int s = (int)blockIdx.x / a.heads, h = (int)blockIdx.x - s * a.heads, b = (int)blockIdx.y;
   const int tid = (int)threadIdx.x;
-  // device metadata is clamped to what the lookup row addresses (never out of the pool)
-  const int len = (int)min(ldg(a.attend_lengths + b), (uint32_t)(a.max_rows - 1)) + 1;
-  const uint32_t w_raw = ldg(a.write_index + b);
-  const int w_idx = w_raw < (uint32_t)a.max_rows ? (int)w_raw : -1;
   const int r0 = s * kAttnSplitRows;
+  // Device metadata (one memory round trip), clamped to what the lookup row addresses (never out of the pool).
+  const uint32_t len_raw = ldg(a.attend_lengths + b);
+  const uint32_t w_raw = ldg(a.write_index + b);
+  const int pos_raw = a.positions != nullptr ? ldg(a.positions + b) : 0;
+  const float* kbase = row_ptr(a, b, h, min(r0, a.max_rows - 1), 0);
+  const int len = (int)min(len_raw, (uint32_t)(a.max_rows - 1)) + 1;
+  const int w_idx = w_raw < (uint32_t)a.max_rows ? (int)w_raw : -1;
+  const int pos = min(max(pos_raw, 0), a.table_rows - 1);
   const int r1 = min(len, r0 + kAttnSplitRows);
   const int64_t bh = (int64_t)b * a.heads + h;
   float* dst = part + (bh * splits + s) * kPart;
-  if (s == 0 && w_idx >= 0) {
-    // the new row into the pool (its readers in this launch take it from k_new / v_new)
-    const int64_t qoff = (int64_t)b * a.in_stride + (int64_t)h * kD;
-    for (int i = tid; i < 2 * kD; i += kThreads) {
-      const int kv = i / kD, d = i % kD;
-      float v;
-      if (kv == 0 && a.positions != nullptr) {
-        const int pos = min(max(ldg(a.positions + b), 0), a.table_rows - 1);
-        v = rope_elem(k_new + qoff, a.cos_t + (int64_t)pos * kD, a.sin_t + (int64_t)pos * kD, d);
-      } else {
-        v = ldg((kv ? v_new : k_new) + qoff + d);
-      }
-      row_ptr(a, b, h, w_idx, kv)[d] = v;
-    }
-  }
   if (r0 >= r1) {  // nothing to attend in this split: an empty partial
     if (tid == 0) {
       publish(dst + kD, -__builtin_huge_valf());
@@ -315,8 +322,19 @@ __global__ void __launch_bounds__(kThreads) k_attn_partial(PagedArgs a, const fl
     }
     for (int d = tid; d < kD; d += kThreads) publish(dst + d, 0.0f);
   } else {
-    split_partial(a, q, k_new, v_new, scale, w_idx, bh, b, h, r0, r1, sc, red, vsum,
+    split_partial(a, q, k_new, v_new, scale, w_idx, pos, b, h, r0, r1, kbase, kbase + a.kv_stride, sc, red, vsum,
                   splits == 1 ? out + bh * kD : nullptr, dst);
+  }
+  if (s == 0 && w_idx >= 0 && tid < 2 * kD) {
+    // the new row into the pool (its readers in this launch take it from k_new / v_new)
+    const int64_t qoff = (int64_t)b * a.in_stride + (int64_t)h * kD;
+    const int kv = tid / kD, d = tid % kD;
+    float v;
+    if (kv == 0 && a.positions != nullptr)
+      v = rope_elem(k_new + qoff, a.cos_t + (int64_t)pos * kD, a.sin_t + (int64_t)pos * kD, d);
+    else
+      v = ldg((kv ? v_new : k_new) + qoff + d);
+    row_ptr(a, b, h, w_idx, kv)[d] = v;
   }
   if (splits == 1 || counters == nullptr) return;
   __builtin_amdgcn_s_waitcnt(0);  // this thread's partial stores done before the count
@@ -363,12 +381,15 @@ hipError_t launch_paged_attention(const PagedAttention& p, hipStream_t s) {
   a.sin_t = p.sin_table;
   a.table_rows = p.table_rows;
   const int splits = (p.max_attend + kAttnSplitRows - 1) / kAttnSplitRows;
-  const dim3 grid((unsigned)(splits > 0 ? splits : 1), (unsigned)p.heads, (unsigned)p.rows);
+  // The heads of a split side by side: their rows are neighbours in memory.
+  const int ns = splits > 0 ? splits : 1;
+  if ((int64_t)p.heads * ns > INT32_MAX) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(p.heads * ns), (unsigned)p.rows);
   UOCR_LAUNCH("attn_partial", k_attn_partial, grid, dim3(kThreads), 0, s, a, p.q, p.k_new, p.v_new, p.scale,
-              p.workspace, (int)grid.x, p.counters, p.out);
-  if (grid.x > 1 && p.counters == nullptr)
+              p.workspace, ns, p.counters, p.out);
+  if (ns > 1 && p.counters == nullptr)
     UOCR_LAUNCH("attn_combine", k_attn_combine, dim3((unsigned)p.heads, (unsigned)p.rows), dim3(kD), 0, s,
-                p.workspace, (int)grid.x, p.heads, p.out);
+                p.workspace, ns, p.heads, p.out);
   return hipGetLastError();
 }
 
