@@ -109,3 +109,14 @@ def test_replays_and_streams(oracle) -> None:
     torch.cuda.synchronize()
     for i in range(2):
         assert all(bits_equal(n(o), want[i]) for o in got[i])
+
+
+def test_routing_launches_agree(oracle) -> None:
+    """The served router's two sets of routing launches (one token apart) route the same tokens alike."""
+    layer = oracle.make_layer(7, E=64, H=1280, F=128, topk=6, int8=True)
+    moe = moe_for(layer)
+    x = _x(1400, 1280)
+    out, ids, wts = (n(v) for v in moe(x, routing=True))
+    few, ids_few, wts_few = (n(v) for v in moe(x[:1399].contiguous(), routing=True))
+    assert np.array_equal(ids[:1399], ids_few) and bits_equal(wts[:1399], wts_few)
+    assert bits_equal(out[:1399], few)

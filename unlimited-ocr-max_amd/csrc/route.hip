@@ -878,7 +878,7 @@ __global__ void __launch_bounds__(kCombineThreads) k_combine(float* __restrict__
 hipError_t launch_logits(float* logits, const float* x, int64_t ldx, const float* router, int T, int E, int H,
                          uint16_t* xb, hipStream_t s, int32_t* zero, int nzero) {
   if (T <= 0) return hipSuccess;
-  if (H == 20 * kWave && E == 64 && T >= 2048) {
+  if (H == 20 * kWave && E == 64 && T >= kRingTokens) {
     // every XCD an equal share of the token blocks (those past T return at once)
     const int ntb = (T + 31) / 32;
     const dim3 grid((unsigned)(kXcds * ((ntb + kXcds - 1) / kXcds) * ((E + 15) / 16)));

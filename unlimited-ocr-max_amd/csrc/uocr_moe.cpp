@@ -1295,11 +1295,11 @@ int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden, co
   const PrefillBufs d = carve_prefill(c, L, T);
   const int E = (int)L->num_experts, H = (int)L->hidden, F = (int)L->ffn, Fs = (int)L->shared_ffn;
 
-  // routing (E <= 64 here): below 2048 tokens one launch computes the logits, the top-k and
+  // routing (E <= 64 here): below 2048 tokens (kRingTokens for the served router) one launch computes the logits, the top-k and
   // per-workgroup counts; above, the logits tiles share router rows over more tokens and the
   // top-k runs in its own launch
   hipError_t e = hipSuccess;
-  if (T < 2048) {
+  if (T < (H == 1280 && E == 64 ? kRingTokens : 2048)) {
     e = launch_logits_topk_group(d.logits, d.xb, x, H, L->router, (int)T, E, H, (int)L->top_k, L->renormalize, d.ids,
                                  d.wts, BM, d.g, d.hist, s);
   } else {
