@@ -90,3 +90,14 @@ def test_special_values(oracle) -> None:
     got, want = n(ops.dense_bf16_qmv(t(x), t(w))), oracle.dense_bf16_qmv_chunked(x, w)
     assert np.isnan(got[3]).all() and np.isinf(got[2]).all()
     assert bits_equal(got[[0, 1, 2, 4, 5]], want[[0, 1, 2, 4, 5]])
+
+
+@pytest.mark.parametrize("topk", [2, 12])
+@pytest.mark.parametrize("b", [15, 16, 33, 64])
+def test_layer_groups_from_the_ids(oracle, b, topk) -> None:
+    """From 16 rows on the routed GEMVs find their rows among the ids (more than 512 of them at 64 x 12)."""
+    layer = oracle.make_layer(b + topk, E=64, H=128, F=64 if b % 2 else 128, topk=topk, int8=False, std=0.05,
+                              router_std=0.3)
+    x = np.random.default_rng(b).standard_normal((b, 128)).astype(np.float32)
+    want, _, _ = oracle.moe_decode_exact(x, layer)
+    assert bits_equal(n(moe_for(layer).decode_rows(t(x))), want)

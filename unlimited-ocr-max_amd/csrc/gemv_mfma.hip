@@ -254,15 +254,16 @@ __device__ __forceinline__ void kblocked_chain(const GemvArgs& a, int p, int n0,
 }
 
 // The rows of a tile: lane l's row of each 4-row tile (padded rows repeat the
-// last real one and are not stored) and its activation pointer.
-template <WKind W, int C, int NT>
-__device__ __forceinline__ void tile_rows(const GemvArgs& a, const int32_t* rows, int t0, int cnt, int (&rowv)[NT],
+// last real one and are not stored) and its activation pointer.  ROUTED: lane
+// i's `row` is row i of up to 64, else the rows are their own numbers.
+template <WKind W, int C, int NT, bool ROUTED>
+__device__ __forceinline__ void tile_rows(const GemvArgs& a, int row, int t0, int cnt, int (&rowv)[NT],
                                           const float* (&xp)[NT]) {
   const int l = lane_id();
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int rr = t0 + min(4 * t + (l & 3), cnt - 1);
-    rowv[t] = rows != nullptr ? ldg(rows + rr) : rr;
+    rowv[t] = ROUTED ? __builtin_amdgcn_ds_bpermute(rr << 2, row) : rr;
     xp[t] = a.x + (int64_t)(rowv[t] / a.x_div) * a.ldx + 4 * (l % C >> 2);
   }
 }
@@ -280,18 +281,18 @@ __device__ __forceinline__ void store_rows(const GemvArgs& a, int n0, int cnt, c
     }
 }
 
-// A workgroup's waves on one row tile (cnt <= 4 NT rows from t0) of a routed
-// expert: wave w takes projection w % NPROJ of column block cb0 + w / NPROJ,
+// A workgroup's waves on one row tile (cnt <= 4 NT rows from t0 of the 64 that
+// the lanes' `row` hold) of a routed expert: wave w takes projection w % NPROJ of column block cb0 + w / NPROJ,
 // all chunks.
 template <WKind W, int NPROJ, int NT>
-__device__ __forceinline__ void routed_tile(const GemvArgs& a, int e, int t0, int cnt, int cb0, char* lds) {
+__device__ __forceinline__ void routed_tile(const GemvArgs& a, int e, int rows, int t0, int cnt, int cb0, char* lds) {
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int l = lane_id();
   const int p = w % NPROJ;
   const int n0 = (cb0 + w / NPROJ) * kWave;
   int rowv[NT];
   const float* xp[NT];
-  tile_rows<W, kWave, NT>(a, a.rows.group_rows, t0, cnt, rowv, xp);
+  tile_rows<W, kWave, NT, true>(a, rows, t0, cnt, rowv, xp);
   f32x4 acc[NT];
   zero(acc);
   char* stage = lds + w * kStageBytes;
@@ -331,7 +332,7 @@ __device__ __forceinline__ void dense_tile(const GemvArgs& a, int t0, int cnt, i
   const int p = w % NPROJ, q = w / NPROJ, Q = (int)(blockDim.x >> 6) / NPROJ;
   int rowv[NT];
   const float* xp[NT];
-  tile_rows<kBf16KBlocked, C, NT>(a, nullptr, t0, cnt, rowv, xp);
+  tile_rows<kBf16KBlocked, C, NT, false>(a, 0, t0, cnt, rowv, xp);
   f32x4 unused[NT];
   constexpr int U = kWave / C;
   const int units = (a.nchunks + U - 1) / U;
@@ -354,27 +355,86 @@ __device__ __forceinline__ void dense_tile(const GemvArgs& a, int t0, int cnt, i
   }
 }
 
-// The routed part of a launch: workgroup wg takes group wg / per_group and the
-// kMfmaWaves / NPROJ column blocks from (wg % per_group) * that many on.
+// Group g of a decode step's routed rows: the g-th expert that has rows, and
+// those, ascending.  Row i's expert is ids[i], each token's ids differ, so an
+// expert has at most one row a token (64).  Lane i's `row` becomes row i; the
+// return value is their number, 0 past the last group.  list: 64 words of the
+// wave's LDS (its stage, idle until its first tile).
+__device__ __forceinline__ int group_of_ids(const int32_t* ids, int nr, int g, int* list, int& e, int& row) {
+  constexpr int kBatch = 8;  // loads in flight
+  const int l = lane_id();
+  int id[kBatch];
+  auto load = [&](int i0) {
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) id[j] = ldg(ids + min(i0 + j * kWave + l, nr - 1));
+  };
+  uint32_t lo = 0u, hi = 0u;
+  for (int i0 = 0; i0 < nr; i0 += kBatch * kWave) {
+    load(i0);
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {  // (past the last row: a repeat of it)
+      lo |= id[j] < 32 ? 1u << (id[j] & 31) : 0u;
+      hi |= id[j] < 32 ? 0u : 1u << (id[j] & 31);
+    }
+  }
+  const uint64_t used = ((uint64_t)tree_or(hi) << 32) | tree_or(lo);
+  const uint64_t nth = __ballot(((used >> l) & 1ull) != 0ull && lanes_below(used) == g);
+  if (nth == 0ull) return 0;
+  e = (int)__builtin_ctzll(nth);
+  int cnt = 0;
+  for (int i0 = 0; i0 < nr; i0 += kBatch * kWave) {
+    if (nr > kBatch * kWave) load(i0);
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      const int i = i0 + j * kWave + l;
+      const bool mine = i < nr && id[j] == e;
+      const uint64_t m = __ballot(mine);
+      const int at = cnt + lanes_below(m);
+      if (mine && at < kWave) list[at] = i;
+      cnt += __builtin_popcountll(m);
+    }
+  }
+  cnt = min(cnt, kWave);
+  __builtin_amdgcn_wave_barrier();
+  row = list[min(l, cnt - 1)];
+  return cnt;
+}
+
+// The routed part of a launch: workgroup wg takes group wg / per and the
+// kMfmaWaves / NPROJ column blocks from (wg % per) * that many on.  With
+// rows.ids a workgroup finds its group among the ids itself: one round trip to
+// memory instead of the three dependent ones of the group tables, and no
+// grouping launch before.
 template <WKind W, int NPROJ>
 __device__ __forceinline__ void routed_part(const GemvArgs& a, int wg, char* lds) {
   constexpr int CB = kMfmaWaves / NPROJ;
+  const int l = lane_id();
   const int per = ((a.N + kWave - 1) / kWave + CB - 1) / CB;
   const int g = wg / per;
-  if (g >= ldc(a.rows.n_groups)) return;
   const int cb0 = (wg - g * per) * CB;
-  const int e = ldc(a.rows.group_expert + g);
-  const int r0 = ldc(a.rows.group_start + g), r1 = ldc(a.rows.group_start + g + 1);
-  for (int t = r0; t < r1; t += 16) {
-    const int cnt = min(16, r1 - t);
-    if (cnt <= 4)
-      routed_tile<W, NPROJ, 1>(a, e, t, cnt, cb0, lds);
-    else if (cnt <= 8)
-      routed_tile<W, NPROJ, 2>(a, e, t, cnt, cb0, lds);
-    else if (cnt <= 12)
-      routed_tile<W, NPROJ, 3>(a, e, t, cnt, cb0, lds);
-    else
-      routed_tile<W, NPROJ, 4>(a, e, t, cnt, cb0, lds);
+  int e = 0, r0 = 0, n = 0, row = 0;
+  if (a.rows.ids != nullptr) {
+    n = group_of_ids(a.rows.ids, a.rows.nids, g, (int*)(lds + (threadIdx.x >> 6) * kStageBytes), e, row);
+  } else {
+    if (g >= ldc(a.rows.n_groups)) return;
+    e = ldc(a.rows.group_expert + g);
+    r0 = ldc(a.rows.group_start + g);
+    n = ldc(a.rows.group_start + g + 1) - r0;
+  }
+  for (int c0 = 0; c0 < n; c0 += kWave) {
+    if (a.rows.ids == nullptr) row = ldg(a.rows.group_rows + r0 + min(c0 + l, n - 1));
+    const int nc = min(n - c0, kWave);
+    for (int t = 0; t < nc; t += 16) {
+      const int cnt = min(16, nc - t);
+      if (cnt <= 4)
+        routed_tile<W, NPROJ, 1>(a, e, row, t, cnt, cb0, lds);
+      else if (cnt <= 8)
+        routed_tile<W, NPROJ, 2>(a, e, row, t, cnt, cb0, lds);
+      else if (cnt <= 12)
+        routed_tile<W, NPROJ, 3>(a, e, row, t, cnt, cb0, lds);
+      else
+        routed_tile<W, NPROJ, 4>(a, e, row, t, cnt, cb0, lds);
+    }
   }
 }
 
@@ -437,7 +497,7 @@ __global__ void __launch_bounds__(kMfmaWaves* kWave) k_dense_whole(GemvArgs a) {
   const int cnt = min(4 * NT, a.rows.identity - d.t0);
   int rowv[NT];
   const float* xp[NT];
-  tile_rows<kBf16KBlocked, kWave, NT>(a, nullptr, d.t0, cnt, rowv, xp);
+  tile_rows<kBf16KBlocked, kWave, NT, false>(a, 0, d.t0, cnt, rowv, xp);
   f32x4 acc[NT];
   zero(acc);
   kblocked_chain<kWave, NT, false>(a, 0, n0, xp, 0, a.nchunks, acc, nullptr);

@@ -433,12 +433,6 @@ __device__ __forceinline__ uint64_t same_key_lanes(int key, int bits) {
   return m;
 }
 
-// Set bits of m below this lane.
-__device__ __forceinline__ int lanes_below(uint64_t m) {
-  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
-
 // Groups R rows by clamped expert id, stably: a group holds its rows in row
 // order.  `idof(r)` returns row r's raw id.  One workgroup of up to 16 waves
 // and E <= blockDim.x; `hist` is LDS of (waves x E) ints, `part` of 3 x 16.
@@ -716,7 +710,7 @@ __global__ void __launch_bounds__(kRouteWaves * 64) k_logits_topk(
   const int rows = nt * topk;
   for (int r = tid; r < rows; r += kRouteWaves * kWave) atomicAdd(&cnt[clamp_expert(ids_lds[r], E)], 1);
   __syncthreads();
-  if (tid < E) stg(hist + (int64_t)b * E + tid, cnt[tid]);
+  if (hist != nullptr && tid < E) stg(hist + (int64_t)b * E + tid, cnt[tid]);
 }
 
 constexpr int kScatterRows = 256;  // rows ranked at once (a pass per 256 rows of a block)
@@ -950,14 +944,27 @@ hipError_t launch_topk_group(const float* logits, int T, int E, int topk, int re
 
 int fused_route_blocks(int T) { return (T + kFusedTokens - 1) / kFusedTokens; }
 
+bool logits_topk_ok(int E, int H, int topk) {
+  return E <= 64 && H % kWave == 0 && H <= kLogitsMaxH && topk <= 64;
+}
+
+hipError_t launch_logits_topk(float* logits, uint16_t* xb, const float* x, int64_t ldx, const float* router, int T,
+                              int E, int H, int topk, int renorm, int32_t* ids32, float* wts, int32_t* hist,
+                              hipStream_t s) {
+  if (T <= 0) return hipSuccess;
+  if (!logits_topk_ok(E, H, topk)) return hipErrorInvalidValue;
+  UOCR_LAUNCH("logits_topk", k_logits_topk, dim3(fused_route_blocks(T)), dim3(kRouteWaves * kWave), 0, s, logits, xb, x,
+              ldx, router, T, E, H, topk, renorm, ids32, wts, hist);
+  return hipGetLastError();
+}
+
 hipError_t launch_logits_topk_group(float* logits, uint16_t* xb, const float* x, int64_t ldx, const float* router,
                                     int T, int E, int H, int topk, int renorm, int32_t* ids32, float* wts, int bm,
                                     const GroupTables& g, int32_t* hist, hipStream_t s) {
   if (T <= 0) return hipSuccess;
-  if (E > 64 || H % kWave != 0 || H > kLogitsMaxH || topk > 64) return hipErrorInvalidValue;
+  const hipError_t e = launch_logits_topk(logits, xb, x, ldx, router, T, E, H, topk, renorm, ids32, wts, hist, s);
+  if (e != hipSuccess) return e;
   const int blocks = fused_route_blocks(T);
-  UOCR_LAUNCH("logits_topk", k_logits_topk, dim3(blocks), dim3(kRouteWaves * kWave), 0, s, logits, xb, x, ldx,
-              router, T, E, H, topk, renorm, ids32, wts, hist);
   UOCR_LAUNCH("group_scatter", k_group_scatter_hist, dim3(blocks), dim3(256), 0, s, ids32, T, E, topk, bm, blocks,
               kFusedTokens, hist, g);
   return hipGetLastError();

@@ -294,6 +294,11 @@ __device__ __forceinline__ uint32_t tree_or(uint32_t v) {
 }
 
 
+// Set bits of m below this lane.
+__device__ __forceinline__ int lanes_below(uint64_t m) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
 __device__ __forceinline__ int clamp_expert(int32_t key, int E) {
   int e = key;
   e = e < 0 ? 0 : e;

@@ -45,6 +45,10 @@ struct Rows {
   const int32_t* group_start;
   const int32_t* group_rows;
   int identity;
+  // Row i's expert (nids rows, each token's experts distinct) for launch_rows_pair, which then groups them
+  // itself and reads no group tables; null: by the tables.
+  const int32_t* ids;
+  int nids;
 };
 
 struct GemvArgs {
@@ -135,6 +139,11 @@ hipError_t launch_topk_group(const float* logits, int T, int E, int topk, int re
 // per-workgroup counts in one launch (xb as launch_logits), then the
 // grouping.  hist holds fused_route_blocks(T) * E ints of scratch.
 int fused_route_blocks(int T);
+// Its first launch alone (hist may be null): E <= 64, H a multiple of 64 and at most 2048, topk <= 64.
+bool logits_topk_ok(int E, int H, int topk);
+hipError_t launch_logits_topk(float* logits, uint16_t* xb, const float* x, int64_t ldx, const float* router, int T,
+                              int E, int H, int topk, int renorm, int32_t* ids32, float* wts, int32_t* hist,
+                              hipStream_t s);
 hipError_t launch_logits_topk_group(float* logits, uint16_t* xb, const float* x, int64_t ldx, const float* router,
                                     int T, int E, int H, int topk, int renorm, int32_t* ids32, float* wts, int bm,
                                     const GroupTables& g, int32_t* hist, hipStream_t s);
