@@ -5,8 +5,8 @@
 // are dequantised with the reference's prefill numerics, w = bf16_rne(f32(q) *
 // scale) (unlimited_ocr_max/kernels/moe_int8.mojo:340, the int8_dequant_expert
 // values), activations rounded to bf16, and v_mfma_f32_32x32x16_bf16
-// accumulates in fp32.  The gate/up launch fuses SwiGLU into its epilogue and
-// writes h in bf16, already packed in group order, which is the down launch's
+// accumulates in fp32.  The gate/up tiles fuse SwiGLU into their epilogue and
+// write h in bf16, already packed in group order, which is the down tiles'
 // A operand.  The shared experts (K-blocked bf16) ride in the same launches as
 // extra tiles with every token as a row.
 //
