@@ -13,11 +13,11 @@
 // Two kernels share the tiling: the LDS-staged one (16-byte aligned weights,
 // the product path) and the fragment-load one (weights at any alignment);
 // both run the same MFMA sequence on the same values, so they give the same
-// bits.  On gfx950 the int8 dequantisation (a conversion, a multiply and half
-// a pack per weight, once per row tile) issues in turn with the MFMAs on a
-// SIMD -- a second wave does not overlap them -- so the int8 kernels are
-// bounded by that issue time; the tiles are sized to spread each dequantised
-// weight over as many rows as the expert has (up to 128).
+// bits.  The int8 dequantisation (a conversion, a multiply and half a pack per
+// weight, once per row tile) takes about as many issue cycles as the MFMAs of a
+// 128-row tile, and runs under them only where it stands between them in a
+// wave's order; the tiles are sized to spread each dequantised weight over as
+// many rows as the expert has (up to 128).
 #include <algorithm>
 #include <atomic>
 
