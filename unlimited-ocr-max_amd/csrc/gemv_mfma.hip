@@ -30,6 +30,15 @@
 
 namespace uocr {
 
+// The byte offset, from a wave's first column, of 16-byte piece `piece` of the
+// wave's column `col` (0 .. 63), or of the last of the `cols` columns from the
+// first one on (rows rowb bytes apart, at most 2^17).  The column is clamped
+// before it is multiplied: a matrix may hold more bytes than an int counts, the
+// wave's 64 columns do not.
+__host__ __device__ int rows_offset(int col, int cols, int rowb, int piece) {
+  return (col < cols ? col : cols - 1) * rowb + 16 * piece;
+}
+
 namespace {
 
 // A stage is 64 x 128 bytes of weights: 128 k of int8, 64 k of bf16.
@@ -144,7 +153,8 @@ __device__ __forceinline__ void rows_chain(const GemvArgs& a, int p, int e, int 
   const int64_t rowb = (int64_t)a.K * (W == kInt8Rows ? 1 : 2);
   const char* base = (const char*)a.p[p].w + ((int64_t)e * a.N + n0) * rowb;
   // load i's lane offset: column n0 + 8 i + l / 8 (past N: the last column)
-  const int off0 = (l >> 3) * (int)rowb + 16 * (l & 7), off_last = (a.N - 1 - n0) * (int)rowb + 16 * (l & 7);
+  const int off0 = (l >> 3) * (int)rowb + 16 * (l & 7);
+  const int off_last = rows_offset(kWave - 1, a.N - n0, (int)rowb, l & 7);
   const float* sp = W == kInt8Rows ? a.p[p].s + ((int64_t)e * a.N + n) * a.nchunks : nullptr;
   i32x4 wn[8], wv[8];
   f32x4 xn[NT][XV], x[NT][XV], part[NT];

@@ -94,6 +94,7 @@ hipError_t launch_gemv_pair(const GemvArgs& routed, int max_groups, const GemvAr
 // (gemv_mfma.hip): 16-byte aligned weights and activations, 128-element int8
 // groups, K a multiple of 64 (the _ok checks).
 constexpr int kMfmaWaves = 4;
+__host__ __device__ int rows_offset(int col, int cols, int rowb, int piece);
 bool rows_pair_ok(const GemvArgs& routed, const GemvArgs& shared, int nproj);
 bool rows_routed_ok(const GemvArgs& a);
 bool rows_dense_ok(const GemvArgs& a);
