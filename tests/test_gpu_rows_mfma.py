@@ -101,3 +101,20 @@ def test_layer_groups_from_the_ids(oracle, b, topk) -> None:
     x = np.random.default_rng(b).standard_normal((b, 128)).astype(np.float32)
     want, _, _ = oracle.moe_decode_exact(x, layer)
     assert bits_equal(n(moe_for(layer).decode_rows(t(x))), want)
+
+
+@pytest.mark.parametrize("rows", [1, 3, 20])
+def test_no_k(rows) -> None:
+    """Sums over no k are zero, at every size of call."""
+    import torch
+
+    from uocr_moe import ops
+
+    x = torch.empty((rows, 0), device="cuda:0")
+    for n_ in (40, 20000):
+        w = torch.empty((0, n_, 16), dtype=torch.bfloat16, device="cuda:0")
+        out = torch.full((rows, n_), float("nan"), device="cuda:0")
+        assert not n(ops.dense_bf16_qmv(x, w, out=out)).any()
+    ids = torch.arange(rows, dtype=torch.int32, device="cuda:0") % 3
+    out = torch.full((rows, 70), float("nan"), device="cuda:0")
+    assert not n(ops.moe_bf16_qmv(x, ids, torch.empty((3, 70, 0), dtype=torch.bfloat16, device="cuda:0"), out=out)).any()

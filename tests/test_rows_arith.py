@@ -3,13 +3,21 @@
 ``rows_offset`` is the kernel's own lane offset into a wave's 64 weight columns, compiled for the host too.  It
 is compared with exact integers over the widths that the ops admit, a matrix of more than 2 GiB among them;
 the 32-bit product of an unclamped column fails the same comparison.
+
+``rows_routed_ok`` and ``rows_dense_ok`` say which calls these kernels take.  A call without any k is not one of
+them: their loops read at least one step, and a plan of no chunks divides by their number.
 """
 
 from __future__ import annotations
 
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
+
+from conftest import PKG_DIR
 
 
 def _internal(symbol: str, restype, *argtypes):
@@ -42,3 +50,52 @@ def test_the_unclamped_product_fails() -> None:
     """From 2 GiB a matrix its last column's offset is negative and would be taken."""
     wrong = [s for s in SHAPES if any(_unclamped(c, *s, 0) != min(c, s[0] - 1) * s[1] for c in range(64))]
     assert (262144, 16384) in wrong and (32769, 65536) in wrong and (129280, 2560) not in wrong
+
+
+class _Rows(ctypes.Structure):
+    _fields_ = [("n_groups", ctypes.c_void_p), ("group_expert", ctypes.c_void_p), ("group_start", ctypes.c_void_p),
+                ("group_rows", ctypes.c_void_p), ("identity", ctypes.c_int), ("ids", ctypes.c_void_p),
+                ("nids", ctypes.c_int)]
+
+
+class _Proj(ctypes.Structure):
+    _fields_ = [("w", ctypes.c_void_p), ("s", ctypes.c_void_p)]
+
+
+class _GemvArgs(ctypes.Structure):
+    """``GemvArgs`` of ``csrc/uocr_kernels.h``."""
+
+    _fields_ = [("out", ctypes.c_void_p), ("ldo", ctypes.c_int64), ("x", ctypes.c_void_p), ("ldx", ctypes.c_int64),
+                ("x_div", ctypes.c_int), ("p", _Proj * 2), ("kind", ctypes.c_int), ("E", ctypes.c_int),
+                ("N", ctypes.c_int), ("K", ctypes.c_int), ("gsize", ctypes.c_int), ("nchunks", ctypes.c_int),
+                ("vec", ctypes.c_int), ("batch", ctypes.c_int), ("rows", _Rows)]
+
+
+INT8_ROWS, BF16_ROWS, BF16_KBLOCKED = 0, 1, 2
+
+
+def _takes(kind: int, K: int, rows: int = 4, N: int = 64, x: int = 0, gsize: int = 128) -> bool:
+    a = _GemvArgs(x=x, ldx=K, x_div=1, kind=kind, E=1, N=N, K=K, gsize=gsize, nchunks=-(-K // 128), vec=1)
+    if kind == BF16_KBLOCKED:
+        a.rows.identity = rows
+        check = _internal("_ZN4uocr13rows_dense_okERKNS_8GemvArgsE", ctypes.c_bool, ctypes.POINTER(_GemvArgs))
+    else:
+        a.rows.n_groups = 256
+        check = _internal("_ZN4uocr14rows_routed_okERKNS_8GemvArgsE", ctypes.c_bool, ctypes.POINTER(_GemvArgs))
+    return check(ctypes.byref(a))
+
+
+@pytest.mark.parametrize("kind", [INT8_ROWS, BF16_ROWS, BF16_KBLOCKED])
+def test_a_call_without_k_is_not_taken(kind) -> None:
+    assert _takes(kind, 128) and _takes(kind, 1280)
+    assert not _takes(kind, 0)
+
+
+def test_dense_call_without_k_returns() -> None:
+    """Rows, columns and no k: an error without a GPU (none is visible to the child), never a signal."""
+    code = ("import ctypes\nfrom uocr_moe import _lib\n"
+            "err = ctypes.create_string_buffer(256)\n"
+            "rc = _lib.load().uocr_dense_bf16_qmv(None, 3, 64, None, 3, 0, None, 0, 64, 16, 1, None, err, 256)\n"
+            "assert rc != 0 and err.value")
+    env = {**os.environ, "PYTHONPATH": str(PKG_DIR), "HIP_VISIBLE_DEVICES": "-1", "ROCR_VISIBLE_DEVICES": "-1"}
+    assert subprocess.run([sys.executable, "-c", code], env=env, timeout=300).returncode == 0

@@ -526,6 +526,7 @@ size_t split_lds(const GemvArgs& a, int nproj, int nt, int c = kWave) {
 }  // namespace
 
 static bool rows_mfma_ok(const GemvArgs& a) {
+  if (a.K <= 0) return false;  // no stage to load; the VALU kernels store the empty sums
   if (!a.vec || (reinterpret_cast<uintptr_t>(a.x) & 15u) != 0 || a.ldx % 4 || a.K > (1 << 16)) return false;
   if (a.kind == kInt8Rows) return a.gsize == kChunk && a.K % kChunk == 0;
   return a.K % 64 == 0;
