@@ -91,6 +91,12 @@ def test_a_call_without_k_is_not_taken(kind) -> None:
     assert not _takes(kind, 0)
 
 
+def test_dense_rows_beyond_a_grid_are_not_taken() -> None:
+    """A workgroup of 256 threads to 32 rows: 2^29 rows would make a grid of 2^32 threads."""
+    assert _takes(BF16_KBLOCKED, 64, rows=1 << 28)
+    assert not _takes(BF16_KBLOCKED, 64, rows=1 << 29)
+
+
 def test_dense_call_without_k_returns() -> None:
     """Rows, columns and no k: an error without a GPU (none is visible to the child), never a signal."""
     code = ("import ctypes\nfrom uocr_moe import _lib\n"

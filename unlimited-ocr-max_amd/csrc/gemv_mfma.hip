@@ -577,8 +577,13 @@ hipError_t launch_rows_routed(const GemvArgs& a, int max_groups, hipStream_t s) 
   return hipGetLastError();
 }
 
+// A launch has a workgroup per row group, and a grid at most 2^32 threads (of narrow outputs, 256 for 32 rows:
+// beyond kMaxDenseRows the VALU kernel's workgroups go over all rows).
+static constexpr int kMaxDenseRows = 1 << 28;
+
 bool rows_dense_ok(const GemvArgs& a) {
-  return a.kind == kBf16KBlocked && a.rows.n_groups == nullptr && rows_mfma_ok(a) && split_lds(a, 1, 1) <= kMaxLds;
+  return a.kind == kBf16KBlocked && a.rows.n_groups == nullptr && a.rows.identity <= kMaxDenseRows &&
+         rows_mfma_ok(a) && split_lds(a, 1, 1) <= kMaxLds;
 }
 
 // How a dense launch is cut: C columns a wave, `waves` of a workgroup on one
