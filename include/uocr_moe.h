@@ -308,7 +308,11 @@ int uocr_moe_decode_stack(float* out, const float* x, int64_t rows, int64_t hidd
  * path).  x fp32 [T, H] -> out fp32 [T, H].  The top-k experts of every token
  * run as a grouped GEMM on the bf16 matrix cores: int8 weights dequantised to
  * bf16_rne(f32(q)*scale) (the reference's prefill values), activations
- * rounded to bf16, fp32 accumulation.  H, F, Fs multiples of 128. */
+ * rounded to bf16, fp32 accumulation.  H, F, Fs multiples of 128.  Calls that
+ * overlap in time must not share a workspace (nor, with workspace == NULL, a
+ * stream's own one across captured graphs): their tables, rows and control
+ * words overwrite each other.  The one in-kernel wait is bounded (about a
+ * second), and a call whose wait ran out writes NaN to all of `out`. */
 int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden,
                      const uocr_moe_layer* layer, int32_t* expert_ids, float* expert_weights,
                      void* workspace, size_t workspace_bytes, void* stream, char* err, size_t errlen);

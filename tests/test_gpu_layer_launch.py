@@ -120,3 +120,16 @@ def test_routing_launches_agree(oracle) -> None:
     few, ids_few, wts_few = (n(v) for v in moe(x[:1399].contiguous(), routing=True))
     assert np.array_equal(ids[:1399], ids_few) and bits_equal(wts[:1399], wts_few)
     assert bits_equal(out[:1399], few)
+
+
+@pytest.mark.parametrize("T", [40, 6000])
+def test_a_wait_without_an_end_is_nan(oracle, monkeypatch, T) -> None:
+    """The down tiles' wait, forced to give up from the host (a limit of 0 polls; every workgroup still exits):
+    the call writes NaN everywhere, and the next one on the same workspace is right again."""
+    moe, other = _pair(oracle, "many", True)
+    x = _x(T, 256)
+    ws = moe.workspace(T, True)
+    monkeypatch.setenv("UOCR_MOE_SPIN_LIMIT", "0")
+    assert np.isnan(n(moe(x, workspace=ws))).all()
+    monkeypatch.delenv("UOCR_MOE_SPIN_LIMIT")
+    assert bits_equal(n(moe(x, workspace=ws)), n(other(x)))

@@ -820,17 +820,31 @@ __device__ __forceinline__ void lds_step(f32x16 (&acc)[NACT][2], const char* st,
 }
 
 constexpr int kCtlLine = 32;  // words between control words
-// The control words of a tile (below): its list's ticket counter, and the
-// finished gate/up tiles.
+// The control words of a tile (below): its list's ticket counter, the
+// finished gate/up tiles, and the word that a wait without an end sets.
 struct PhaseCtl {
   int32_t* ticket;
   int32_t* done;
+  int32_t* failed;
+  uint32_t spin;  // polls a wait may take
 };
 __device__ __forceinline__ int32_t agent_load(const int32_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ int32_t agent_add(int32_t* p, int32_t v) {
   return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Waits (one thread) until `need` gate/up tiles of counter `dep` have finished,
+// at most ctl.spin polls: then, or once another wait has given up, it goes on
+// with `failed` set, and the layer's combine writes NaN.  A limit of 0 fails
+// every wait, even one whose tiles are done (the host's test of this path).
+__device__ __forceinline__ void wait_rows(const PhaseCtl& ctl, int dep, int need) {
+  for (uint32_t spin = ctl.spin;; --spin) {
+    if (spin != 0u && agent_load(ctl.done + dep * kCtlLine) >= need) return;
+    if (spin == 0u || ((spin & 1023u) == 0u && agent_load(ctl.failed) != 0)) break;
+    __builtin_amdgcn_s_sleep(1);
+  }
+  __hip_atomic_store(ctl.failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // One tile whose rows fill NACT 32-row blocks: only those blocks' A rows are
 // loaded and computed.  A gate/up tile (NPROJ 2) counts itself finished once
@@ -971,9 +985,9 @@ __device__ __forceinline__ int lds_tile(const GemmProblem& P, const TileRef& t, 
   issue_b(0);
   if constexpr (NPROJ == 1) {
     // The wait ends: every gate/up tile has been taken by a running workgroup,
-    // and none of those waits for anything.
-    if (threadIdx.x == 0)
-      while (agent_load(ctl.done + t.dep * kCtlLine) < t.need) __builtin_amdgcn_s_sleep(1);
+    // and none of those waits for anything.  It is bounded for a launch whose
+    // control words another call overwrote.
+    if (threadIdx.x == 0) wait_rows(ctl, t.dep, t.need);
     asm volatile("s_barrier" ::: "memory");
   }
 #pragma unroll
@@ -1333,9 +1347,11 @@ __device__ __forceinline__ int shared_tile(const GemmProblem& b, const TileRef& 
 // The control words of a launch, zeroed before it, each on a line of its own
 // (agent-scope accesses skip the L2, and those of one line queue at the
 // memory): per phase (gate/up, down) and XCD a ticket counter and, after it,
-// the list's length + 1 once a workgroup has planned it; then the finished
-// gate/up tiles of each expert's rows and of each shared row tile.
-constexpr int kCtlDone = 2 * kXcds * kCtlLine;
+// the list's length + 1 once a workgroup has planned it; then the word that a
+// failed wait sets, and the finished gate/up tiles of each expert's rows and of
+// each shared row tile.
+constexpr int kCtlFailed = 2 * kXcds * kCtlLine;
+constexpr int kCtlDone = kCtlFailed + kCtlLine;
 constexpr int kCtlSharedDep = 64;  // num_experts <= 64
 
 // Thread 0's value in every wave (the LDS word lies in the rings, idle between tiles).
@@ -1359,19 +1375,19 @@ __device__ __forceinline__ int broadcast(int v, char* lds) {
 // T = 291 92 -> 96 us, T = 64 87 -> 93).
 constexpr int kPatience = 16;
 template <int NP, bool STEAL, typename PlanFn, typename RunFn>
-__device__ __forceinline__ void walk(int32_t* ctl, char* lds, PlanFn&& plan, RunFn&& run) {
+__device__ __forceinline__ void walk(int32_t* ctl, uint32_t spin, char* lds, PlanFn&& plan, RunFn&& run) {
   int32_t* lists = ctl + (NP == 2 ? 0 : kXcds) * kCtlLine;
   const int own = (int)blockIdx.x % kXcds;
   uint32_t unseen = (1u << kXcds) - 1;  // lists this workgroup has not run to their end
   for (int x = own;;) {
-    const PhaseCtl pc{lists + x * kCtlLine, ctl + kCtlDone};
+    const PhaseCtl pc{lists + x * kCtlLine, ctl + kCtlDone, ctl + kCtlFailed, spin};
     int v = 0;
     if (threadIdx.x == 0) v = agent_add(pc.ticket, 1);
     const int n = plan(x);
     int it = broadcast(v, lds);
     if (it == 0 && threadIdx.x == 0)
       __hip_atomic_store(pc.ticket + 1, n + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    while (it < n) it = run(it, pc);
+    while ((uint32_t)it < (uint32_t)n) it = run(it, pc);  // (an overwritten counter may give any value)
     if (!STEAL && NP == 1) return;
     unseen &= ~(1u << x);
     if (threadIdx.x < kWave) {
@@ -1395,7 +1411,7 @@ __device__ __forceinline__ void walk(int32_t* ctl, char* lds, PlanFn&& plan, Run
 // routed and the shared problem (a down tile waits for all of its rows').
 template <WKind W0, int NP>
 __device__ __forceinline__ void walk_balanced(const GemmProblem& a, const GemmProblem& b, int colsa, int colsb,
-                                              int32_t* ctl, char* lds_stages) {
+                                              int32_t* ctl, uint32_t spin, char* lds_stages) {
   constexpr int bn = kWRowsWg / NP;
   constexpr int BMA = kLdsBM<W0>, BMB = kLdsBM<kBf16KBlocked>;
   Seq q;
@@ -1441,13 +1457,13 @@ __device__ __forceinline__ void walk_balanced(const GemmProblem& a, const GemmPr
     t.need = colsb;
     return shared_tile<NP>(b, t, lds_stages, pc);
   };
-  walk<NP, true>(ctl, lds_stages, plan, run);
+  walk<NP, true>(ctl, spin, lds_stages, plan, run);
 }
 
 // The by-class placement's list of XCD x.
 template <WKind W0, int NP>
 __device__ __forceinline__ void walk_classes(const GemmProblem& a, const GemmProblem& b, int colsa, int colsb,
-                                             int32_t* ctl, char* lds_stages) {
+                                             int32_t* ctl, uint32_t spin, char* lds_stages) {
   constexpr int bn = kWRowsWg / NP;
   constexpr int BMA = kLdsBM<W0>, BMB = kLdsBM<kBf16KBlocked>;
   const int ntr = (b.N + bn - 1) / bn;  // the shared problem's column tiles, in every K range
@@ -1491,7 +1507,7 @@ __device__ __forceinline__ void walk_classes(const GemmProblem& a, const GemmPro
     t.need = colsb;
     return shared_tile<NP>(b, t, lds_stages, pc);
   };
-  walk<NP, false>(ctl, lds_stages, plan, run);
+  walk<NP, false>(ctl, spin, lds_stages, plan, run);
 }
 
 // Gate/up (a, b) and down (c, d) of the routed and the shared experts in one
@@ -1505,16 +1521,16 @@ __device__ __forceinline__ void walk_classes(const GemmProblem& a, const GemmPro
 // 112 -> 109, T = 4096 371 -> 349, bf16 T = 1531 250 -> 224.
 template <WKind W0, bool BAL>
 __global__ void __launch_bounds__(kGThreads, kWgPerCu) k_moe_layer(GemmProblem a, GemmProblem b, GemmProblem c,
-                                                                   GemmProblem d, int32_t* ctl) {
+                                                                   GemmProblem d, int32_t* ctl, uint32_t spin) {
   extern __shared__ __attribute__((aligned(16))) char lds_stages[];
   constexpr int bn = kWRowsWg / 2;
   const int colsa = (a.N + bn - 1) / bn, colsb = (b.N + bn - 1) / bn;
   if constexpr (BAL) {
-    walk_balanced<W0, 2>(a, b, colsa, colsb, ctl, lds_stages);
-    walk_balanced<W0, 1>(c, d, colsa, colsb, ctl, lds_stages);
+    walk_balanced<W0, 2>(a, b, colsa, colsb, ctl, spin, lds_stages);
+    walk_balanced<W0, 1>(c, d, colsa, colsb, ctl, spin, lds_stages);
   } else {
-    walk_classes<W0, 2>(a, b, colsa, colsb, ctl, lds_stages);
-    walk_classes<W0, 1>(c, d, colsa, colsb, ctl, lds_stages);
+    walk_classes<W0, 2>(a, b, colsa, colsb, ctl, spin, lds_stages);
+    walk_classes<W0, 1>(c, d, colsa, colsb, ctl, spin, lds_stages);
   }
 }
 
@@ -1555,16 +1571,18 @@ int64_t tile_bound(const GemmProblem& routed, const GemmProblem& shared, int sha
 // phase is the larger one where ffn is near hidden).
 template <WKind W0>
 hipError_t launch_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn, const GemmProblem& sdn,
-                        int32_t* ctl, hipStream_t s) {
+                        int32_t* ctl, uint32_t spin, hipStream_t s) {
   constexpr size_t lds = kLdsBytes<W0>;
   int grid = 0;
   const hipError_t e = moe_layer_grid<W0>(&grid);
   if (e != hipSuccess) return e;
   const int64_t rounds2 = std::min(2 * (int64_t)grid, (int64_t)kMaxUnits);
   if (tile_bound<W0>(gu, sgu, 1) > rounds2 || tile_bound<W0>(dn, sdn, parts_of(sdn)) > rounds2)
-    UOCR_LAUNCH("gemm_layer", (k_moe_layer<W0, true>), dim3(grid), dim3(kGThreads), lds, s, gu, sgu, dn, sdn, ctl);
+    UOCR_LAUNCH("gemm_layer", (k_moe_layer<W0, true>), dim3(grid), dim3(kGThreads), lds, s, gu, sgu, dn, sdn, ctl,
+                spin);
   else
-    UOCR_LAUNCH("gemm_layer", (k_moe_layer<W0, false>), dim3(grid), dim3(kGThreads), lds, s, gu, sgu, dn, sdn, ctl);
+    UOCR_LAUNCH("gemm_layer", (k_moe_layer<W0, false>), dim3(grid), dim3(kGThreads), lds, s, gu, sgu, dn, sdn, ctl,
+                spin);
   return hipGetLastError();
 }
 
@@ -1621,6 +1639,8 @@ int moe_layer_ctl_words(int64_t tokens) {
          kCtlLine * (kCtlSharedDep + (int)((tokens + kLdsBM<kBf16KBlocked> - 1) / kLdsBM<kBf16KBlocked>));
 }
 
+int moe_layer_failed_word() { return kCtlFailed; }
+
 // 16-byte aligned weights, at most kMaxScaleGroups int8 groups a row, and a
 // lane per routed group in the placement's plan; the fragment-load kernel
 // takes the rest, a launch per phase.
@@ -1630,10 +1650,10 @@ bool moe_layer_ok(const GemmProblem& gu, const GemmProblem& dn, bool vec) {
 }
 
 hipError_t launch_moe_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn,
-                            const GemmProblem& sdn, int32_t* ctl, hipStream_t s) {
+                            const GemmProblem& sdn, int32_t* ctl, uint32_t spin, hipStream_t s) {
   if (!gemm_shapes_ok(gu, sgu) || !gemm_shapes_ok(dn, sdn)) return hipErrorInvalidValue;
-  return gu.kind == kInt8Rows ? launch_layer<kInt8Rows>(gu, sgu, dn, sdn, ctl, s)
-                              : launch_layer<kBf16Rows>(gu, sgu, dn, sdn, ctl, s);
+  return gu.kind == kInt8Rows ? launch_layer<kInt8Rows>(gu, sgu, dn, sdn, ctl, spin, s)
+                              : launch_layer<kBf16Rows>(gu, sgu, dn, sdn, ctl, spin, s);
 }
 
 // One phase of the layer with the fragment-load kernel (64-row tiles).

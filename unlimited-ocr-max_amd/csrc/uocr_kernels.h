@@ -155,9 +155,11 @@ hipError_t launch_route_small(const float* logits, int T, int E, int topk, int r
 
 // out[t, n] = fma-chain over j of wts[t*k+j] * y[row(t*k+j), n] from 0, then
 // + shared[r][t, n] for r < shared_parts in turn (parts T x H floats apart).
-// row(i) = inv ? inv[i] : i.  shared may be null.
+// row(i) = inv ? inv[i] : i.  shared may be null.  NaN throughout if *failed
+// (may be null) is not 0.
 hipError_t launch_combine(float* out, const float* y, int64_t ldy, const float* wts, const int32_t* inv,
-                          const float* shared, int T, int H, int topk, hipStream_t s, int shared_parts = 1);
+                          const float* shared, int T, int H, int topk, hipStream_t s, int shared_parts = 1,
+                          const int32_t* failed = nullptr);
 
 // ---- int8 dequantisation and the prefill grouped GEMM (gemm.hip) ----
 
@@ -202,11 +204,14 @@ struct GemmProblem {
 //
 // Gate/up and down of a layer in one launch: dn and sdn read what gu and sgu
 // write.  ctl: moe_layer_ctl_words(tokens) words, zero before the launch (the
-// grouping's launch clears them).  moe_layer_ok: what it takes.
+// grouping's launch clears them).  A down tile waits for its rows at most
+// spin_limit polls, then the launch goes on with word moe_layer_failed_word()
+// set.  moe_layer_ok: what it takes.
 int moe_layer_ctl_words(int64_t tokens);
+int moe_layer_failed_word();
 bool moe_layer_ok(const GemmProblem& gu, const GemmProblem& dn, bool vec);
 hipError_t launch_moe_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn,
-                            const GemmProblem& sdn, int32_t* ctl, hipStream_t s);
+                            const GemmProblem& sdn, int32_t* ctl, uint32_t spin_limit, hipStream_t s);
 // One phase, weights at any alignment, with the same bits.
 hipError_t launch_gemm_pair(const GemmProblem& routed, const GemmProblem& shared, hipStream_t s);
 // The K ranges to cut the shared problem into for this pair (1 or 2).

@@ -830,17 +830,20 @@ static bool fused_eligible(const uocr_moe_layer* L, int64_t B) {
   return lay.lds_bytes <= kMaxLds;
 }
 
-// Polls per bounded wait of the persistent kernel: 2^16 (tens of milliseconds;
-// healthy waits take microseconds).  UOCR_MOE_SPIN_LIMIT overrides it, so a
-// test can make the waits run out and check the failure path (0: every wait
-// fails at once, even one whose data is there).
-static uint32_t fused_spin_limit() {
+// Polls per bounded wait of the persistent decode kernel, 2^16 (tens of
+// milliseconds; healthy waits take microseconds), and of the prefill layer's,
+// 2^20 (about a second; a healthy one ends with another workgroup's tile).
+// UOCR_MOE_SPIN_LIMIT overrides both, so a test can make the waits run out and
+// check the failure path (0: every wait fails at once, even one whose data is
+// there).
+constexpr uint32_t kDecodeSpin = 1u << 16, kPrefillSpin = 1u << 20;
+static uint32_t spin_limit(uint32_t limit) {
   const char* env = std::getenv("UOCR_MOE_SPIN_LIMIT");
   if (env != nullptr) {
     const long v = std::strtol(env, nullptr, 10);
     if (v >= 0 && v <= (1L << 30)) return (uint32_t)v;
   }
-  return 1u << 16;
+  return limit;
 }
 
 static FusedLayerW fused_weights(const uocr_moe_layer* L) {
@@ -905,7 +908,7 @@ static FusedArgs fused_args(const uocr_moe_layer* L, int64_t B, const FusedLayou
   a.early_shared = B <= kFusedEarlySharedRows ? 1 : 0;
   a.defer_down = B <= kFusedEarlySharedRows ? 1 : 0;
   a.m_h = magic(a.H);
-  a.spin_limit = fused_spin_limit();
+  a.spin_limit = spin_limit(kDecodeSpin);
   return a;
 }
 
@@ -1390,13 +1393,14 @@ int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden, co
   sdn.kparts = gemm_shared_parts(dn, sdn);
   sdn.part_stride = T * H;
   if (moe_layer_ok(gu, dn, vec && aligned16(ws))) {
-    e = launch_moe_layer(gu, sgu, dn, sdn, d.g.ctl, s);
+    e = launch_moe_layer(gu, sgu, dn, sdn, d.g.ctl, spin_limit(kPrefillSpin), s);
   } else {
     e = launch_gemm_pair(gu, sgu, s);
     if (e == hipSuccess) e = launch_gemm_pair(dn, sdn, s);
   }
   if (e == hipSuccess)
-    e = launch_combine(out, d.y, H, d.wts, d.g.inv, d.sh, (int)T, H, (int)L->top_k, s, sdn.kparts);
+    e = launch_combine(out, d.y, H, d.wts, d.g.inv, d.sh, (int)T, H, (int)L->top_k, s, sdn.kparts,
+                       d.g.ctl + moe_layer_failed_word());
   if (e == hipSuccess && expert_ids) e = hipMemcpyAsync(expert_ids, d.ids, R * sizeof(int32_t), hipMemcpyDeviceToDevice, s);
   if (e == hipSuccess && expert_weights)
     e = hipMemcpyAsync(expert_weights, d.wts, R * sizeof(float), hipMemcpyDeviceToDevice, s);
