@@ -80,6 +80,9 @@ __device__ __forceinline__ void rope_pair4(f32x4& lo, f32x4& hi, f32x4 cl, f32x4
     hi[e] = h * ch[e] + l * sh[e];
   }
 }
+// Row i of a split's n, or, past the end, one of its rows: of different ones for
+// neighbouring i, since loads of one line by every lane queue for it.
+__device__ __forceinline__ int live_row(int i, int n) { return i < n ? i : min(i & 15, n - 1); }
 // Four floats of a table row (4-byte aligned).
 __device__ __forceinline__ f32x4 load4(const float* p) {
   return f32x4{ldg(p), ldg(p + 1), ldg(p + 2), ldg(p + 3)};
@@ -154,11 +157,12 @@ __device__ __forceinline__ void split_partial(const PagedArgs& a, const float* _
                                               f32x4 (*vsum)[kD / 4], float* direct, float* dst) {
   const int tid = (int)threadIdx.x;
   // ---- every load of the split first: k (8 lanes per row, a load instruction covering 128 contiguous
-  // bytes of a row) and v (32 lanes per row, a float4 each).  Lanes past the attended rows repeat the
-  // last one's loads (no branch, and no bytes of rows that are not attended); their values are masked
-  // below.  The step's metadata, the pool row's address and q's tables come before and cost one round
-  // trip each, under no other load (8 rows of up to 640 / 1200: 13.4 -> 12.9, 23.5 -> 22.4 us, of which
-  // the bytes are 7 and 14).
+  // bytes of a row) and v (32 lanes per row, a float4 each).  Lanes past the attended rows repeat
+  // attended ones' loads (no branch, and no bytes of rows that are not attended); their values are
+  // masked below.  The step's metadata and the pool row's address are read in one round trip, q's
+  // tables before the keys.  Against reading whole splits, a round trip more (cold pages, us): 1 row of
+  // 16 / 128 / 640 6.4 -> 5.5, 6.9 -> 7.1, 8.4 -> 8.5; 8 rows of 300 / 640 / 1200 11.1 -> 9.9, 16.4 ->
+  // 16.3, 27.8 -> 26.5.  (Lanes that all repeat the last row: 1 row of 16 5.9.)
   const int n = r1 - r0;
   const int sub = tid % kLanesPerRow, rg = tid / kLanesPerRow;
   const int c = tid % (kD / 4), g = tid / (kD / 4);
@@ -180,7 +184,7 @@ __device__ __forceinline__ void split_partial(const PagedArgs& a, const float* _
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int j = 0; j < kKRows; ++j) {
-    const int i = min(rg + j * kRowsPerPass, n - 1);
+    const int i = live_row(rg + j * kRowsPerPass, n);
     const float* kr = (r0 + i == w_idx ? k_new + qoff : kbase + (int64_t)i * a.slot_stride) + sub * 4;
 #pragma unroll
     for (int u = 0; u < 4; ++u) kv[j][u] = *(const UOCR_GLOBAL f32x4*)(kr + 32 * u);
@@ -195,7 +199,7 @@ __device__ __forceinline__ void split_partial(const PagedArgs& a, const float* _
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int j = 0; j < kVRows; ++j) {
-    const int i = min(g + j * kValueGroups, n - 1);
+    const int i = live_row(g + j * kValueGroups, n);
     const float* vr = r0 + i == w_idx ? v_new + qoff : vbase + (int64_t)i * a.slot_stride;
     vv[j] = *(const UOCR_GLOBAL f32x4*)(vr + 4 * c);
   }
@@ -203,7 +207,7 @@ __device__ __forceinline__ void split_partial(const PagedArgs& a, const float* _
   if (rc != nullptr) {
 #pragma unroll
     for (int j = 0; j < kKRows; ++j) {
-      if (r0 + min(rg + j * kRowsPerPass, n - 1) == w_idx) {  // the new row, read unrotated
+      if (r0 + live_row(rg + j * kRowsPerPass, n) == w_idx) {  // the new row, read unrotated
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           cv[u] = load4(rc + sub * 4 + 32 * u);
@@ -301,7 +305,7 @@ __global__ void __launch_bounds__(kThreads, 4) k_attn_partial(PagedArgs a, const
   __shared__ float red[kThreads / 64];
   __shared__ f32x4 vsum[kValueGroups - 1][kD / 4];
   __shared__ uint32_t last;
-  const int s = (int)blockIdx.x / a.heads, h = (int)blockIdx.x - s * a.heads, b = (int)blockIdx.y;
+  const int s = (int)blockIdx.x, h = (int)blockIdx.y, b = (int)blockIdx.z;
   const int tid = (int)threadIdx.x;
   const int r0 = s * kAttnSplitRows;
   // Device metadata (one memory round trip), clamped to what the lookup row addresses (never out of the pool).
@@ -315,6 +319,18 @@ __global__ void __launch_bounds__(kThreads, 4) k_attn_partial(PagedArgs a, const
   const int r1 = min(len, r0 + kAttnSplitRows);
   const int64_t bh = (int64_t)b * a.heads + h;
   float* dst = part + (bh * splits + s) * kPart;
+  if (s == 0 && w_idx >= 0 && tid < 2 * kD) {
+    // the new row into the pool (its readers in this launch take it from k_new / v_new), before the loads:
+    // after them it took 0.3 us more where a request has one split
+    const int64_t qoff = (int64_t)b * a.in_stride + (int64_t)h * kD;
+    const int kv = tid / kD, d = tid % kD;
+    float v;
+    if (kv == 0 && a.positions != nullptr)
+      v = rope_elem(k_new + qoff, a.cos_t + (int64_t)pos * kD, a.sin_t + (int64_t)pos * kD, d);
+    else
+      v = ldg((kv ? v_new : k_new) + qoff + d);
+    row_ptr(a, b, h, w_idx, kv)[d] = v;
+  }
   if (r0 >= r1) {  // nothing to attend in this split: an empty partial
     if (tid == 0) {
       publish(dst + kD, -__builtin_huge_valf());
@@ -324,17 +340,6 @@ __global__ void __launch_bounds__(kThreads, 4) k_attn_partial(PagedArgs a, const
   } else {
     split_partial(a, q, k_new, v_new, scale, w_idx, pos, b, h, r0, r1, kbase, kbase + a.kv_stride, sc, red, vsum,
                   splits == 1 ? out + bh * kD : nullptr, dst);
-  }
-  if (s == 0 && w_idx >= 0 && tid < 2 * kD) {
-    // the new row into the pool (its readers in this launch take it from k_new / v_new)
-    const int64_t qoff = (int64_t)b * a.in_stride + (int64_t)h * kD;
-    const int kv = tid / kD, d = tid % kD;
-    float v;
-    if (kv == 0 && a.positions != nullptr)
-      v = rope_elem(k_new + qoff, a.cos_t + (int64_t)pos * kD, a.sin_t + (int64_t)pos * kD, d);
-    else
-      v = ldg((kv ? v_new : k_new) + qoff + d);
-    row_ptr(a, b, h, w_idx, kv)[d] = v;
   }
   if (splits == 1 || counters == nullptr) return;
   __builtin_amdgcn_s_waitcnt(0);  // this thread's partial stores done before the count
@@ -381,10 +386,9 @@ hipError_t launch_paged_attention(const PagedAttention& p, hipStream_t s) {
   a.sin_t = p.sin_table;
   a.table_rows = p.table_rows;
   const int splits = (p.max_attend + kAttnSplitRows - 1) / kAttnSplitRows;
-  // The heads of a split side by side: their rows are neighbours in memory.
+  // (The heads of a split side by side, neighbours in memory, took 0.2 us more at 1 row and 0.4 at 8 of 640.)
   const int ns = splits > 0 ? splits : 1;
-  if ((int64_t)p.heads * ns > INT32_MAX) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)(p.heads * ns), (unsigned)p.rows);
+  const dim3 grid((unsigned)ns, (unsigned)p.heads, (unsigned)p.rows);
   UOCR_LAUNCH("attn_partial", k_attn_partial, grid, dim3(kThreads), 0, s, a, p.q, p.k_new, p.v_new, p.scale,
               p.workspace, ns, p.counters, p.out);
   if (ns > 1 && p.counters == nullptr)
