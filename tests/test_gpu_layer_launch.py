@@ -1,4 +1,4 @@
-"""The prefill layer's one GEMM launch (gate/up tiles, then down tiles that wait for their rows).
+"""The prefill layer's one GEMM launch (gate/up tiles, then down tiles that wait for their rows), and a phase alone.
 
 Weights at an odd address take the fragment-load kernel, a launch per phase and the same bits, so the two
 paths are compared bit for bit: at the edges of the tiles (32-row blocks, 64- and 128-row tiles), with one
@@ -19,15 +19,17 @@ SHAPES = {  # experts, hidden, ffn (top 2, 2 shared experts)
     "small": (8, 256, 128),
     "many": (64, 256, 256),
     "one": (1, 128, 128),
+    "fine gate/up": (8, 1152, 256),  # at int8 group 64: 18 groups a row, down 4
+    "fine down": (8, 256, 1152),
 }
 
 
-def _pair(oracle, shape: str, int8: bool):
+def _pair(oracle, shape: str, int8: bool, group: int = 128):
     """A layer with aligned weights, and the same one with its gate stack at an odd (2-byte for bf16) address."""
     from uocr_moe import MoE
 
     E, H, F = SHAPES[shape]
-    layer = oracle.make_layer(5, E=E, H=H, F=F, topk=min(2, E), int8=int8, std=0.05, router_std=0.1)
+    layer = oracle.make_layer(5, E=E, H=H, F=F, topk=min(2, E), int8=int8, group=group, std=0.05, router_std=0.1)
     moe = moe_for(layer)
     w = layer_weights(layer)
     gate = w["experts.gate_proj"]
@@ -133,3 +135,18 @@ def test_a_wait_without_an_end_is_nan(oracle, monkeypatch, T) -> None:
     assert np.isnan(n(moe(x, workspace=ws))).all()
     monkeypatch.delenv("UOCR_MOE_SPIN_LIMIT")
     assert bits_equal(n(moe(x, workspace=ws)), n(other(x)))
+
+
+@pytest.mark.parametrize("T", [1, 33, 130, 700, 2100])
+@pytest.mark.parametrize(("shape", "staged"), [("fine gate/up", "gemm_down"), ("fine down", "gemm_gateup")])
+def test_one_phase_staged(oracle, shape, staged, T) -> None:
+    """More than 16 int8 groups a row in one phase: only that phase leaves the LDS-staged kernel."""
+    from uocr_moe import _lib
+
+    moe, other = _pair(oracle, shape, True, group=64)
+    x = _x(T, SHAPES[shape][1])
+    _lib.timing_begin(16)
+    got = n(moe(x))
+    names = [name for name, _ in _lib.timing_end(16)]
+    assert staged in names and sum(name.startswith("gemm_") for name in names) == 2
+    assert bits_equal(got, n(other(x)))

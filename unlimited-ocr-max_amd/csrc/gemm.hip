@@ -850,14 +850,16 @@ __device__ __forceinline__ void wait_rows(const PhaseCtl& ctl, int dep, int need
 // loaded and computed.  A gate/up tile (NPROJ 2) counts itself finished once
 // its h rows are past the L2; a down tile waits for its h rows after its first
 // weights are on their way.  Returns the workgroup's next ticket of the list,
-// taken during the last step.
-template <int BM, WKind W, int NPROJ, int NACT>
+// taken during the last step.  JOINT: both phases run in one launch (else
+// neither the count, nor the wait, nor h past the L2 is needed).
+template <int BM, WKind W, int NPROJ, int NACT, bool JOINT>
 __device__ __forceinline__ int lds_tile(const GemmProblem& P, const TileRef& t, char* lds, const PhaseCtl& ctl) {
   using St = Stage<BM, W>;
   using Rg = Ring<BM, W, NACT>;
   constexpr int NB = St::kBLoads, NA = Rg::kALoads, NL = NB + NA;
   constexpr int RB = St::kBRowBytes;
   constexpr int RPL = 1024 / RB;  // weight rows per load
+  constexpr bool kGives = JOINT && NPROJ == 2, kTakes = JOINT && NPROJ == 1;
   // The thread index passes through an empty asm per tile, so that what is
   // derived from it (addresses, swizzles) is computed in the tile and not
   // hoisted out of the tile loop, where it held about 40 VGPRs across every
@@ -954,7 +956,7 @@ __device__ __forceinline__ int lds_tile(const GemmProblem& P, const TileRef& t, 
     char* st = lds + Rg::kB * St::kBBytes + (s % Rg::kA) * Rg::kAStep;
     const char* base = (const char*)(P.a + (k0 + s) * BK);
 #pragma unroll
-    for (int i = 0; i < NA; ++i) dma16<NPROJ == 1 ? kAgentLoad : 0>(base + lane_offset(aoff[i]), st + (4 * i + w) * 1024);
+    for (int i = 0; i < NA; ++i) dma16<kTakes ? kAgentLoad : 0>(base + lane_offset(aoff[i]), st + (4 * i + w) * 1024);
   };
 
   f32x16 acc[NACT][2];
@@ -983,7 +985,7 @@ __device__ __forceinline__ int lds_tile(const GemmProblem& P, const TileRef& t, 
   constexpr int LA = Rg::kA - 1, LB = Rg::kB - 1;
   static_assert(LA >= 1 && LB <= 2 && (LA == LB || LA == LB - 1), "ring depth");
   issue_b(0);
-  if constexpr (NPROJ == 1) {
+  if constexpr (kTakes) {
     // The wait ends: every gate/up tile has been taken by a running workgroup,
     // and none of those waits for anything.  It is bounded for a launch whose
     // control words another call overwrote.
@@ -1021,12 +1023,12 @@ __device__ __forceinline__ int lds_tile(const GemmProblem& P, const TileRef& t, 
     Q.outf += t.e * P.part_stride;
     store_tile<32 * NACT, NPROJ>(Q, t, acc, w, m, h);
   } else {
-    store_tile<32 * NACT, NPROJ, NPROJ == 2>(P, t, acc, w, m, h);
+    store_tile<32 * NACT, NPROJ, kGives>(P, t, acc, w, m, h);
   }
-  if constexpr (NPROJ == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // h is past the L2
+  if constexpr (kGives) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // h is past the L2
   lds_barrier();
   ticket = __builtin_amdgcn_readfirstlane(*(const int*)lds);
-  if (NPROJ == 2 && threadIdx.x == 0) (void)agent_add(ctl.done + t.dep * kCtlLine, 1);
+  if (kGives && threadIdx.x == 0) (void)agent_add(ctl.done + t.dep * kCtlLine, 1);
   lds_barrier();
   return ticket;
 }
@@ -1323,25 +1325,25 @@ __device__ __forceinline__ Sched make_sched(const GemmProblem& a, const GemmProb
 }
 
 // A routed or shared tile by its active 32-row blocks.
-template <WKind W0, int NP>
+template <WKind W0, int NP, bool JOINT>
 __device__ __forceinline__ int routed_tile(const GemmProblem& a, const TileRef& t, char* lds, const PhaseCtl& pc) {
   constexpr int BMA = kLdsBM<W0>;
   const int nact = (t.rows + 31) >> 5;
   if constexpr (BMA == 128) {
-    if (nact == 4) return lds_tile<BMA, W0, NP, 4>(a, t, lds, pc);
-    if (nact == 3) return lds_tile<BMA, W0, NP, 3>(a, t, lds, pc);
+    if (nact == 4) return lds_tile<BMA, W0, NP, 4, JOINT>(a, t, lds, pc);
+    if (nact == 3) return lds_tile<BMA, W0, NP, 3, JOINT>(a, t, lds, pc);
   } else {
     static_assert(BMA == 64, "64- or 128-row tiles");
   }
-  if (nact == 2) return lds_tile<BMA, W0, NP, 2>(a, t, lds, pc);
-  return lds_tile<BMA, W0, NP, 1>(a, t, lds, pc);
+  if (nact == 2) return lds_tile<BMA, W0, NP, 2, JOINT>(a, t, lds, pc);
+  return lds_tile<BMA, W0, NP, 1, JOINT>(a, t, lds, pc);
 }
-template <int NP>
+template <int NP, bool JOINT>
 __device__ __forceinline__ int shared_tile(const GemmProblem& b, const TileRef& t, char* lds, const PhaseCtl& pc) {
   constexpr int BMB = kLdsBM<kBf16KBlocked>;
   static_assert(BMB == 64, "64-row shared tiles");
-  if (t.rows > 32) return lds_tile<BMB, kBf16KBlocked, NP, 2>(b, t, lds, pc);
-  return lds_tile<BMB, kBf16KBlocked, NP, 1>(b, t, lds, pc);
+  if (t.rows > 32) return lds_tile<BMB, kBf16KBlocked, NP, 2, JOINT>(b, t, lds, pc);
+  return lds_tile<BMB, kBf16KBlocked, NP, 1, JOINT>(b, t, lds, pc);
 }
 
 // The control words of a launch, zeroed before it, each on a line of its own
@@ -1374,7 +1376,7 @@ __device__ __forceinline__ int broadcast(int v, char* lds) {
 // taken by its own workgroups, which have it planned (taking them at once:
 // T = 291 92 -> 96 us, T = 64 87 -> 93).
 constexpr int kPatience = 16;
-template <int NP, bool STEAL, typename PlanFn, typename RunFn>
+template <int NP, bool STEAL, bool JOINT, typename PlanFn, typename RunFn>
 __device__ __forceinline__ void walk(int32_t* ctl, uint32_t spin, char* lds, PlanFn&& plan, RunFn&& run) {
   int32_t* lists = ctl + (NP == 2 ? 0 : kXcds) * kCtlLine;
   const int own = (int)blockIdx.x % kXcds;
@@ -1388,7 +1390,7 @@ __device__ __forceinline__ void walk(int32_t* ctl, uint32_t spin, char* lds, Pla
     if (it == 0 && threadIdx.x == 0)
       __hip_atomic_store(pc.ticket + 1, n + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     while ((uint32_t)it < (uint32_t)n) it = run(it, pc);  // (an overwritten counter may give any value)
-    if (!STEAL && NP == 1) return;
+    if (!STEAL && !(JOINT && NP == 2)) return;
     unseen &= ~(1u << x);
     if (threadIdx.x < kWave) {
       // a bit per list whose tickets have not run past its length, or whose length is not known yet
@@ -1409,7 +1411,7 @@ __device__ __forceinline__ void walk(int32_t* ctl, uint32_t spin, char* lds, Pla
 
 // The balanced placement's list of XCD x.  cols: gate/up column tiles of the
 // routed and the shared problem (a down tile waits for all of its rows').
-template <WKind W0, int NP>
+template <WKind W0, int NP, bool JOINT>
 __device__ __forceinline__ void walk_balanced(const GemmProblem& a, const GemmProblem& b, int colsa, int colsb,
                                               int32_t* ctl, uint32_t spin, char* lds_stages) {
   constexpr int bn = kWRowsWg / NP;
@@ -1443,7 +1445,7 @@ __device__ __forceinline__ void walk_balanced(const GemmProblem& a, const GemmPr
       t.e = __builtin_amdgcn_readlane(q.e, g);
       t.dep = t.e;
       t.need = colsa * ((count + BMA - 1) / BMA);
-      return routed_tile<W0, NP>(a, t, lds_stages, pc);
+      return routed_tile<W0, NP, JOINT>(a, t, lds_stages, pc);
     }
     const int mt = b0 + i / q.ntb;
     const int cr = i - (mt - b0) * q.ntb;  // K range cr / ntr, column tile cr % ntr
@@ -1455,13 +1457,13 @@ __device__ __forceinline__ void walk_balanced(const GemmProblem& a, const GemmPr
     t.rows = min(BMB, b.M - mt * BMB);
     t.dep = kCtlSharedDep + mt;
     t.need = colsb;
-    return shared_tile<NP>(b, t, lds_stages, pc);
+    return shared_tile<NP, JOINT>(b, t, lds_stages, pc);
   };
-  walk<NP, true>(ctl, spin, lds_stages, plan, run);
+  walk<NP, true, JOINT>(ctl, spin, lds_stages, plan, run);
 }
 
 // The by-class placement's list of XCD x.
-template <WKind W0, int NP>
+template <WKind W0, int NP, bool JOINT>
 __device__ __forceinline__ void walk_classes(const GemmProblem& a, const GemmProblem& b, int colsa, int colsb,
                                              int32_t* ctl, uint32_t spin, char* lds_stages) {
   constexpr int bn = kWRowsWg / NP;
@@ -1497,7 +1499,7 @@ __device__ __forceinline__ void walk_classes(const GemmProblem& a, const GemmPro
       TileRef t = class_tile<BMA>(a, qa, nact, it, bn);
       t.dep = t.e;
       t.need *= colsa;
-      return routed_tile<W0, NP>(a, t, lds_stages, pc);
+      return routed_tile<W0, NP, JOINT>(a, t, lds_stages, pc);
     }
     TileRef t = class_tile<BMB>(b, qb, nact, it, bn);
     const int cr = t.n0 / bn;  // K range cr / ntr, column tile cr % ntr
@@ -1505,9 +1507,9 @@ __device__ __forceinline__ void walk_classes(const GemmProblem& a, const GemmPro
     t.n0 = (cr - t.e * ntr) * bn;
     t.dep = kCtlSharedDep + t.pos0 / BMB;
     t.need = colsb;
-    return shared_tile<NP>(b, t, lds_stages, pc);
+    return shared_tile<NP, JOINT>(b, t, lds_stages, pc);
   };
-  walk<NP, false>(ctl, spin, lds_stages, plan, run);
+  walk<NP, false, JOINT>(ctl, spin, lds_stages, plan, run);
 }
 
 // Gate/up (a, b) and down (c, d) of the routed and the shared experts in one
@@ -1526,12 +1528,22 @@ __global__ void __launch_bounds__(kGThreads, kWgPerCu) k_moe_layer(GemmProblem a
   constexpr int bn = kWRowsWg / 2;
   const int colsa = (a.N + bn - 1) / bn, colsb = (b.N + bn - 1) / bn;
   if constexpr (BAL) {
-    walk_balanced<W0, 2>(a, b, colsa, colsb, ctl, spin, lds_stages);
-    walk_balanced<W0, 1>(c, d, colsa, colsb, ctl, spin, lds_stages);
+    walk_balanced<W0, 2, true>(a, b, colsa, colsb, ctl, spin, lds_stages);
+    walk_balanced<W0, 1, true>(c, d, colsa, colsb, ctl, spin, lds_stages);
   } else {
-    walk_classes<W0, 2>(a, b, colsa, colsb, ctl, spin, lds_stages);
-    walk_classes<W0, 1>(c, d, colsa, colsb, ctl, spin, lds_stages);
+    walk_classes<W0, 2, true>(a, b, colsa, colsb, ctl, spin, lds_stages);
+    walk_classes<W0, 1, true>(c, d, colsa, colsb, ctl, spin, lds_stages);
   }
+}
+
+// One phase alone, the other in a launch of its own.
+template <WKind W0, int NP, bool BAL>
+__global__ void __launch_bounds__(kGThreads, kWgPerCu) k_moe_phase(GemmProblem a, GemmProblem b, int32_t* ctl) {
+  extern __shared__ __attribute__((aligned(16))) char lds_stages[];
+  if constexpr (BAL)
+    walk_balanced<W0, NP, false>(a, b, 0, 0, ctl, 0u, lds_stages);
+  else
+    walk_classes<W0, NP, false>(a, b, 0, 0, ctl, 0u, lds_stages);
 }
 
 // Workgroups of the layer's grid: every CU's resident share, a whole number
@@ -1545,7 +1557,9 @@ hipError_t moe_layer_grid(int* grid) {
     int dev = 0, cus = 0, per_cu = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    for (const void* f : {(const void*)k_moe_layer<W0, false>, (const void*)k_moe_layer<W0, true>})
+    for (const void* f : {(const void*)k_moe_layer<W0, false>, (const void*)k_moe_layer<W0, true>,
+                          (const void*)k_moe_phase<W0, 2, false>, (const void*)k_moe_phase<W0, 2, true>,
+                          (const void*)k_moe_phase<W0, 1, false>, (const void*)k_moe_phase<W0, 1, true>})
       if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e == hipSuccess)
       e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_moe_layer<W0, false>, kGThreads, lds);
@@ -1570,14 +1584,40 @@ int64_t tile_bound(const GemmProblem& routed, const GemmProblem& shared, int sha
 // grid (the by-class plan holds kMaxUnits units of a problem; the gate/up
 // phase is the larger one where ffn is near hidden).
 template <WKind W0>
+bool balanced(const GemmProblem& routed, const GemmProblem& shared, int grid) {
+  return tile_bound<W0>(routed, shared, parts_of(shared)) > std::min(2 * (int64_t)grid, (int64_t)kMaxUnits);
+}
+
+template <WKind W0>
+hipError_t launch_phase(const GemmProblem& routed, const GemmProblem& shared, const char* name, int32_t* ctl,
+                        hipStream_t s) {
+  constexpr size_t lds = kLdsBytes<W0>;
+  int grid = 0;
+  const hipError_t e = moe_layer_grid<W0>(&grid);
+  if (e != hipSuccess) return e;
+  const dim3 g(grid), b(kGThreads);
+  if (routed.swiglu) {
+    if (balanced<W0>(routed, shared, grid))
+      UOCR_LAUNCH(name, (k_moe_phase<W0, 2, true>), g, b, lds, s, routed, shared, ctl);
+    else
+      UOCR_LAUNCH(name, (k_moe_phase<W0, 2, false>), g, b, lds, s, routed, shared, ctl);
+  } else {
+    if (balanced<W0>(routed, shared, grid))
+      UOCR_LAUNCH(name, (k_moe_phase<W0, 1, true>), g, b, lds, s, routed, shared, ctl);
+    else
+      UOCR_LAUNCH(name, (k_moe_phase<W0, 1, false>), g, b, lds, s, routed, shared, ctl);
+  }
+  return hipGetLastError();
+}
+
+template <WKind W0>
 hipError_t launch_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn, const GemmProblem& sdn,
                         int32_t* ctl, uint32_t spin, hipStream_t s) {
   constexpr size_t lds = kLdsBytes<W0>;
   int grid = 0;
   const hipError_t e = moe_layer_grid<W0>(&grid);
   if (e != hipSuccess) return e;
-  const int64_t rounds2 = std::min(2 * (int64_t)grid, (int64_t)kMaxUnits);
-  if (tile_bound<W0>(gu, sgu, 1) > rounds2 || tile_bound<W0>(dn, sdn, parts_of(sdn)) > rounds2)
+  if (balanced<W0>(gu, sgu, grid) || balanced<W0>(dn, sdn, grid))
     UOCR_LAUNCH("gemm_layer", (k_moe_layer<W0, true>), dim3(grid), dim3(kGThreads), lds, s, gu, sgu, dn, sdn, ctl,
                 spin);
   else
@@ -1643,10 +1683,11 @@ int moe_layer_failed_word() { return kCtlFailed; }
 
 // 16-byte aligned weights, at most kMaxScaleGroups int8 groups a row, and a
 // lane per routed group in the placement's plan; the fragment-load kernel
-// takes the rest, a launch per phase.
-bool moe_layer_ok(const GemmProblem& gu, const GemmProblem& dn, bool vec) {
-  if (!vec || gu.max_groups > kWave) return false;
-  return gu.kind != kInt8Rows || (gu.groups <= kMaxScaleGroups && dn.groups <= kMaxScaleGroups);
+// takes the rest.  Each phase by itself: at int8 group 64, hidden 1280 and ffn
+// 896, gate/up has 20 groups a row and down 14 (T = 512 / 4096 149 / 570 us
+// with both on the fragment-load kernel, 137 / 495 with gate/up alone).
+bool gemm_staged_ok(const GemmProblem& routed, bool vec) {
+  return vec && routed.max_groups <= kWave && (routed.kind != kInt8Rows || routed.groups <= kMaxScaleGroups);
 }
 
 hipError_t launch_moe_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn,
@@ -1656,16 +1697,25 @@ hipError_t launch_moe_layer(const GemmProblem& gu, const GemmProblem& sgu, const
                               : launch_layer<kBf16Rows>(gu, sgu, dn, sdn, ctl, spin, s);
 }
 
-// One phase of the layer with the fragment-load kernel (64-row tiles).
-hipError_t launch_gemm_pair(const GemmProblem& routed, const GemmProblem& shared, hipStream_t s) {
-  const bool gu = routed.swiglu != 0;
-  const char* name = gu ? "gemm_gateup" : "gemm_down";
+template <WKind W0>
+static hipError_t launch_fragment(const GemmProblem& routed, const GemmProblem& shared, const char* name,
+                                  hipStream_t s) {
+  return routed.swiglu ? launch_moe_gemm<64, W0, 2, false>(routed, shared, s, name)
+                       : launch_moe_gemm<64, W0, 1, false>(routed, shared, s, name);
+}
+
+hipError_t launch_gemm_phase(const GemmProblem& routed, const GemmProblem& shared, bool vec, int32_t* ctl,
+                             hipStream_t s) {
   if (!gemm_shapes_ok(routed, shared)) return hipErrorInvalidValue;
-  if (routed.kind == kInt8Rows)
-    return gu ? launch_moe_gemm<64, kInt8Rows, 2, false>(routed, shared, s, name)
-              : launch_moe_gemm<64, kInt8Rows, 1, false>(routed, shared, s, name);
-  return gu ? launch_moe_gemm<64, kBf16Rows, 2, false>(routed, shared, s, name)
-            : launch_moe_gemm<64, kBf16Rows, 1, false>(routed, shared, s, name);
+  const bool int8 = routed.kind == kInt8Rows;
+  if (!gemm_staged_ok(routed, vec)) {  // 64-row tiles
+    const char* name = routed.swiglu ? "gemm_gateup_any" : "gemm_down_any";
+    return int8 ? launch_fragment<kInt8Rows>(routed, shared, name, s)
+                : launch_fragment<kBf16Rows>(routed, shared, name, s);
+  }
+  const char* name = routed.swiglu ? "gemm_gateup" : "gemm_down";
+  return int8 ? launch_phase<kInt8Rows>(routed, shared, name, ctl, s)
+              : launch_phase<kBf16Rows>(routed, shared, name, ctl, s);
 }
 
 }  // namespace uocr

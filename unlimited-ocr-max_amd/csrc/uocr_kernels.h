@@ -202,18 +202,20 @@ struct GemmProblem {
 // N must be a multiple of 32 and K of 128 (and of the int8 group, itself a
 // multiple of 64); a routed problem has at most 64 groups.
 //
-// Gate/up and down of a layer in one launch: dn and sdn read what gu and sgu
-// write.  ctl: moe_layer_ctl_words(tokens) words, zero before the launch (the
-// grouping's launch clears them).  A down tile waits for its rows at most
-// spin_limit polls, then the launch goes on with word moe_layer_failed_word()
-// set.  moe_layer_ok: what it takes.
+// gemm_staged_ok: the LDS-staged kernels take the problem (vec: every operand is
+// 16-byte aligned).  ctl: moe_layer_ctl_words(tokens) words, zero before a
+// layer's first launch (the grouping's launch clears them).
+bool gemm_staged_ok(const GemmProblem& routed, bool vec);
 int moe_layer_ctl_words(int64_t tokens);
+// Gate/up and down of a layer in one launch, both staged: dn and sdn read what
+// gu and sgu write.  A down tile waits for its rows at most spin_limit polls,
+// then the launch goes on with word moe_layer_failed_word() set.
 int moe_layer_failed_word();
-bool moe_layer_ok(const GemmProblem& gu, const GemmProblem& dn, bool vec);
 hipError_t launch_moe_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn,
                             const GemmProblem& sdn, int32_t* ctl, uint32_t spin_limit, hipStream_t s);
-// One phase, weights at any alignment, with the same bits.
-hipError_t launch_gemm_pair(const GemmProblem& routed, const GemmProblem& shared, hipStream_t s);
+// One phase, staged or with weights at any alignment, with the same bits.
+hipError_t launch_gemm_phase(const GemmProblem& routed, const GemmProblem& shared, bool vec, int32_t* ctl,
+                             hipStream_t s);
 // The K ranges to cut the shared problem into for this pair (1 or 2).
 int gemm_shared_parts(const GemmProblem& routed, const GemmProblem& shared);
 

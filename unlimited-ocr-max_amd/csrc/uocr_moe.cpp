@@ -1392,11 +1392,12 @@ int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden, co
   // launch's longest at T = 512 (down 43 -> 35 us).
   sdn.kparts = gemm_shared_parts(dn, sdn);
   sdn.part_stride = T * H;
-  if (moe_layer_ok(gu, dn, vec && aligned16(ws))) {
+  const bool staged = vec && aligned16(ws);
+  if (gemm_staged_ok(gu, staged) && gemm_staged_ok(dn, staged)) {
     e = launch_moe_layer(gu, sgu, dn, sdn, d.g.ctl, spin_limit(kPrefillSpin), s);
   } else {
-    e = launch_gemm_pair(gu, sgu, s);
-    if (e == hipSuccess) e = launch_gemm_pair(dn, sdn, s);
+    e = launch_gemm_phase(gu, sgu, staged, d.g.ctl, s);
+    if (e == hipSuccess) e = launch_gemm_phase(dn, sdn, staged, d.g.ctl, s);
   }
   if (e == hipSuccess)
     e = launch_combine(out, d.y, H, d.wts, d.g.inv, d.sh, (int)T, H, (int)L->top_k, s, sdn.kparts,
