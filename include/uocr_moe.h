@@ -312,7 +312,8 @@ int uocr_moe_decode_stack(float* out, const float* x, int64_t rows, int64_t hidd
  * overlap in time must not share a workspace (nor, with workspace == NULL, a
  * stream's own one across captured graphs): their tables, rows and control
  * words overwrite each other.  The one in-kernel wait is bounded (about a
- * second), and a call whose wait ran out writes NaN to all of `out`. */
+ * second), and a call whose wait ran out writes NaN to all of `out`
+ * and `expert_weights`. */
 int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden,
                      const uocr_moe_layer* layer, int32_t* expert_ids, float* expert_weights,
                      void* workspace, size_t workspace_bytes, void* stream, char* err, size_t errlen);

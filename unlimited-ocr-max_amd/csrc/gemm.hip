@@ -820,13 +820,18 @@ __device__ __forceinline__ void lds_step(f32x16 (&acc)[NACT][2], const char* st,
 }
 
 constexpr int kCtlLine = 32;  // words between control words
-// The control words of a tile (below): its list's ticket counter, the
-// finished gate/up tiles, and the word that a wait without an end sets.
+// Of a layer's launch: polls a wait may take, and the combine's weights.
+struct Guard {
+  uint32_t spin;
+  int nwts;
+  float* wts;
+};
+// The control words of a tile (below): its list's ticket counter, and the
+// finished gate/up tiles, after the word that a wait without an end sets.
 struct PhaseCtl {
   int32_t* ticket;
   int32_t* done;
-  int32_t* failed;
-  uint32_t spin;  // polls a wait may take
+  Guard guard;
 };
 __device__ __forceinline__ int32_t agent_load(const int32_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -835,16 +840,18 @@ __device__ __forceinline__ int32_t agent_add(int32_t* p, int32_t v) {
   return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // Waits (one thread) until `need` gate/up tiles of counter `dep` have finished,
-// at most ctl.spin polls: then, or once another wait has given up, it goes on
-// with `failed` set, and the layer's combine writes NaN.  A limit of 0 fails
-// every wait, even one whose tiles are done (the host's test of this path).
+// at most guard.spin polls: then, or once another wait has given up, it goes on,
+// with every weight of the combine NaN.  A limit of 0 fails every wait, even one
+// whose tiles are done (the host's test of this path).
 __device__ __forceinline__ void wait_rows(const PhaseCtl& ctl, int dep, int need) {
-  for (uint32_t spin = ctl.spin;; --spin) {
+  int32_t* failed = ctl.done - kCtlLine;
+  for (uint32_t spin = ctl.guard.spin;; --spin) {
     if (spin != 0u && agent_load(ctl.done + dep * kCtlLine) >= need) return;
-    if (spin == 0u || ((spin & 1023u) == 0u && agent_load(ctl.failed) != 0)) break;
+    if (spin == 0u || ((spin & 1023u) == 0u && agent_load(failed) != 0)) break;
     __builtin_amdgcn_s_sleep(1);
   }
-  __hip_atomic_store(ctl.failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (__hip_atomic_exchange(failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 1)
+    for (int i = 0; i < ctl.guard.nwts; ++i) stg(ctl.guard.wts + i, __builtin_nanf(""));
 }
 // One tile whose rows fill NACT 32-row blocks: only those blocks' A rows are
 // loaded and computed.  A gate/up tile (NPROJ 2) counts itself finished once
@@ -1377,12 +1384,12 @@ __device__ __forceinline__ int broadcast(int v, char* lds) {
 // T = 291 92 -> 96 us, T = 64 87 -> 93).
 constexpr int kPatience = 16;
 template <int NP, bool STEAL, bool JOINT, typename PlanFn, typename RunFn>
-__device__ __forceinline__ void walk(int32_t* ctl, uint32_t spin, char* lds, PlanFn&& plan, RunFn&& run) {
+__device__ __forceinline__ void walk(int32_t* ctl, const Guard& guard, char* lds, PlanFn&& plan, RunFn&& run) {
   int32_t* lists = ctl + (NP == 2 ? 0 : kXcds) * kCtlLine;
   const int own = (int)blockIdx.x % kXcds;
   uint32_t unseen = (1u << kXcds) - 1;  // lists this workgroup has not run to their end
   for (int x = own;;) {
-    const PhaseCtl pc{lists + x * kCtlLine, ctl + kCtlDone, ctl + kCtlFailed, spin};
+    const PhaseCtl pc{lists + x * kCtlLine, ctl + kCtlDone, guard};
     int v = 0;
     if (threadIdx.x == 0) v = agent_add(pc.ticket, 1);
     const int n = plan(x);
@@ -1413,7 +1420,7 @@ __device__ __forceinline__ void walk(int32_t* ctl, uint32_t spin, char* lds, Pla
 // routed and the shared problem (a down tile waits for all of its rows').
 template <WKind W0, int NP, bool JOINT>
 __device__ __forceinline__ void walk_balanced(const GemmProblem& a, const GemmProblem& b, int colsa, int colsb,
-                                              int32_t* ctl, uint32_t spin, char* lds_stages) {
+                                              int32_t* ctl, const Guard& guard, char* lds_stages) {
   constexpr int bn = kWRowsWg / NP;
   constexpr int BMA = kLdsBM<W0>, BMB = kLdsBM<kBf16KBlocked>;
   Seq q;
@@ -1459,13 +1466,13 @@ __device__ __forceinline__ void walk_balanced(const GemmProblem& a, const GemmPr
     t.need = colsb;
     return shared_tile<NP, JOINT>(b, t, lds_stages, pc);
   };
-  walk<NP, true, JOINT>(ctl, spin, lds_stages, plan, run);
+  walk<NP, true, JOINT>(ctl, guard, lds_stages, plan, run);
 }
 
 // The by-class placement's list of XCD x.
 template <WKind W0, int NP, bool JOINT>
 __device__ __forceinline__ void walk_classes(const GemmProblem& a, const GemmProblem& b, int colsa, int colsb,
-                                             int32_t* ctl, uint32_t spin, char* lds_stages) {
+                                             int32_t* ctl, const Guard& guard, char* lds_stages) {
   constexpr int bn = kWRowsWg / NP;
   constexpr int BMA = kLdsBM<W0>, BMB = kLdsBM<kBf16KBlocked>;
   const int ntr = (b.N + bn - 1) / bn;  // the shared problem's column tiles, in every K range
@@ -1509,7 +1516,7 @@ __device__ __forceinline__ void walk_classes(const GemmProblem& a, const GemmPro
     t.need = colsb;
     return shared_tile<NP, JOINT>(b, t, lds_stages, pc);
   };
-  walk<NP, false, JOINT>(ctl, spin, lds_stages, plan, run);
+  walk<NP, false, JOINT>(ctl, guard, lds_stages, plan, run);
 }
 
 // Gate/up (a, b) and down (c, d) of the routed and the shared experts in one
@@ -1523,16 +1530,16 @@ __device__ __forceinline__ void walk_classes(const GemmProblem& a, const GemmPro
 // 112 -> 109, T = 4096 371 -> 349, bf16 T = 1531 250 -> 224.
 template <WKind W0, bool BAL>
 __global__ void __launch_bounds__(kGThreads, kWgPerCu) k_moe_layer(GemmProblem a, GemmProblem b, GemmProblem c,
-                                                                   GemmProblem d, int32_t* ctl, uint32_t spin) {
+                                                                   GemmProblem d, int32_t* ctl, Guard guard) {
   extern __shared__ __attribute__((aligned(16))) char lds_stages[];
   constexpr int bn = kWRowsWg / 2;
   const int colsa = (a.N + bn - 1) / bn, colsb = (b.N + bn - 1) / bn;
   if constexpr (BAL) {
-    walk_balanced<W0, 2, true>(a, b, colsa, colsb, ctl, spin, lds_stages);
-    walk_balanced<W0, 1, true>(c, d, colsa, colsb, ctl, spin, lds_stages);
+    walk_balanced<W0, 2, true>(a, b, colsa, colsb, ctl, guard, lds_stages);
+    walk_balanced<W0, 1, true>(c, d, colsa, colsb, ctl, guard, lds_stages);
   } else {
-    walk_classes<W0, 2, true>(a, b, colsa, colsb, ctl, spin, lds_stages);
-    walk_classes<W0, 1, true>(c, d, colsa, colsb, ctl, spin, lds_stages);
+    walk_classes<W0, 2, true>(a, b, colsa, colsb, ctl, guard, lds_stages);
+    walk_classes<W0, 1, true>(c, d, colsa, colsb, ctl, guard, lds_stages);
   }
 }
 
@@ -1541,9 +1548,9 @@ template <WKind W0, int NP, bool BAL>
 __global__ void __launch_bounds__(kGThreads, kWgPerCu) k_moe_phase(GemmProblem a, GemmProblem b, int32_t* ctl) {
   extern __shared__ __attribute__((aligned(16))) char lds_stages[];
   if constexpr (BAL)
-    walk_balanced<W0, NP, false>(a, b, 0, 0, ctl, 0u, lds_stages);
+    walk_balanced<W0, NP, false>(a, b, 0, 0, ctl, Guard{}, lds_stages);
   else
-    walk_classes<W0, NP, false>(a, b, 0, 0, ctl, 0u, lds_stages);
+    walk_classes<W0, NP, false>(a, b, 0, 0, ctl, Guard{}, lds_stages);
 }
 
 // Workgroups of the layer's grid: every CU's resident share, a whole number
@@ -1612,17 +1619,17 @@ hipError_t launch_phase(const GemmProblem& routed, const GemmProblem& shared, co
 
 template <WKind W0>
 hipError_t launch_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn, const GemmProblem& sdn,
-                        int32_t* ctl, uint32_t spin, hipStream_t s) {
+                        int32_t* ctl, const Guard& guard, hipStream_t s) {
   constexpr size_t lds = kLdsBytes<W0>;
   int grid = 0;
   const hipError_t e = moe_layer_grid<W0>(&grid);
   if (e != hipSuccess) return e;
   if (balanced<W0>(gu, sgu, grid) || balanced<W0>(dn, sdn, grid))
     UOCR_LAUNCH("gemm_layer", (k_moe_layer<W0, true>), dim3(grid), dim3(kGThreads), lds, s, gu, sgu, dn, sdn, ctl,
-                spin);
+                guard);
   else
     UOCR_LAUNCH("gemm_layer", (k_moe_layer<W0, false>), dim3(grid), dim3(kGThreads), lds, s, gu, sgu, dn, sdn, ctl,
-                spin);
+                guard);
   return hipGetLastError();
 }
 
@@ -1679,8 +1686,6 @@ int moe_layer_ctl_words(int64_t tokens) {
          kCtlLine * (kCtlSharedDep + (int)((tokens + kLdsBM<kBf16KBlocked> - 1) / kLdsBM<kBf16KBlocked>));
 }
 
-int moe_layer_failed_word() { return kCtlFailed; }
-
 // 16-byte aligned weights, at most kMaxScaleGroups int8 groups a row, and a
 // lane per routed group in the placement's plan; the fragment-load kernel
 // takes the rest.  Each phase by itself: at int8 group 64, hidden 1280 and ffn
@@ -1691,10 +1696,12 @@ bool gemm_staged_ok(const GemmProblem& routed, bool vec) {
 }
 
 hipError_t launch_moe_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn,
-                            const GemmProblem& sdn, int32_t* ctl, uint32_t spin, hipStream_t s) {
+                            const GemmProblem& sdn, int32_t* ctl, uint32_t spin_limit, float* wts, int nwts,
+                            hipStream_t s) {
   if (!gemm_shapes_ok(gu, sgu) || !gemm_shapes_ok(dn, sdn)) return hipErrorInvalidValue;
-  return gu.kind == kInt8Rows ? launch_layer<kInt8Rows>(gu, sgu, dn, sdn, ctl, spin, s)
-                              : launch_layer<kBf16Rows>(gu, sgu, dn, sdn, ctl, spin, s);
+  const Guard guard{spin_limit, nwts, wts};
+  return gu.kind == kInt8Rows ? launch_layer<kInt8Rows>(gu, sgu, dn, sdn, ctl, guard, s)
+                              : launch_layer<kBf16Rows>(gu, sgu, dn, sdn, ctl, guard, s);
 }
 
 template <WKind W0>

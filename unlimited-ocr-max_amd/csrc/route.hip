@@ -832,10 +832,9 @@ __global__ void __launch_bounds__(kCombineThreads) k_combine(float* __restrict__
                                                              int64_t ldy, const float* __restrict__ wts,
                                                              const int32_t* __restrict__ inv,
                                                              const float* __restrict__ shared, int T, int H, int topk,
-                                                             int parts, const int32_t* __restrict__ failed) {
+                                                             int parts) {
   typedef float vec __attribute__((ext_vector_type(W)));
   const int t = (int)blockIdx.x;
-  const bool nan = failed != nullptr && ldc(failed) != 0;
   for (int n = W * (int)threadIdx.x; n < H; n += W * kCombineThreads) {
     vec acc = {};
     // up to kCombineMaxK rows in flight; the fma chain stays in slot order
@@ -864,7 +863,6 @@ __global__ void __launch_bounds__(kCombineThreads) k_combine(float* __restrict__
 #pragma unroll
       for (int c = 0; c < W; ++c) acc[c] = acc[c] + sh[c];
     }
-    if (nan) acc = __builtin_nanf("");
     *(UOCR_GLOBAL vec*)(out + (int64_t)t * H + n) = acc;
   }
 }
@@ -981,17 +979,16 @@ hipError_t launch_route_small(const float* logits, int T, int E, int topk, int r
 }
 
 hipError_t launch_combine(float* out, const float* y, int64_t ldy, const float* wts, const int32_t* inv,
-                          const float* shared, int T, int H, int topk, hipStream_t s, int shared_parts,
-                          const int32_t* failed) {
+                          const float* shared, int T, int H, int topk, hipStream_t s, int shared_parts) {
   if (T <= 0) return hipSuccess;
   if (shared_parts < 1) return hipErrorInvalidValue;
   const auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
   if (H % 4 == 0 && ldy % 4 == 0 && a16(out) && a16(y) && (shared == nullptr || a16(shared)))
     UOCR_LAUNCH("combine", k_combine<4>, dim3(T), dim3(kCombineThreads), 0, s, out, y, ldy, wts, inv, shared, T, H,
-                topk, shared_parts, failed);
+                topk, shared_parts);
   else
     UOCR_LAUNCH("combine", k_combine<1>, dim3(T), dim3(kCombineThreads), 0, s, out, y, ldy, wts, inv, shared, T, H,
-                topk, shared_parts, failed);
+                topk, shared_parts);
   return hipGetLastError();
 }
 

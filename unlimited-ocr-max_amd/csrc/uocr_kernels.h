@@ -155,11 +155,9 @@ hipError_t launch_route_small(const float* logits, int T, int E, int topk, int r
 
 // out[t, n] = fma-chain over j of wts[t*k+j] * y[row(t*k+j), n] from 0, then
 // + shared[r][t, n] for r < shared_parts in turn (parts T x H floats apart).
-// row(i) = inv ? inv[i] : i.  shared may be null.  NaN throughout if *failed
-// (may be null) is not 0.
+// row(i) = inv ? inv[i] : i.  shared may be null.
 hipError_t launch_combine(float* out, const float* y, int64_t ldy, const float* wts, const int32_t* inv,
-                          const float* shared, int T, int H, int topk, hipStream_t s, int shared_parts = 1,
-                          const int32_t* failed = nullptr);
+                          const float* shared, int T, int H, int topk, hipStream_t s, int shared_parts = 1);
 
 // ---- int8 dequantisation and the prefill grouped GEMM (gemm.hip) ----
 
@@ -209,10 +207,11 @@ bool gemm_staged_ok(const GemmProblem& routed, bool vec);
 int moe_layer_ctl_words(int64_t tokens);
 // Gate/up and down of a layer in one launch, both staged: dn and sdn read what
 // gu and sgu write.  A down tile waits for its rows at most spin_limit polls,
-// then the launch goes on with word moe_layer_failed_word() set.
-int moe_layer_failed_word();
+// then the launch goes on and the nwts weights of the
+// combine, wts, become NaN.
 hipError_t launch_moe_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn,
-                            const GemmProblem& sdn, int32_t* ctl, uint32_t spin_limit, hipStream_t s);
+                            const GemmProblem& sdn, int32_t* ctl, uint32_t spin_limit, float* wts, int nwts,
+                            hipStream_t s);
 // One phase, staged or with weights at any alignment, with the same bits.
 hipError_t launch_gemm_phase(const GemmProblem& routed, const GemmProblem& shared, bool vec, int32_t* ctl,
                              hipStream_t s);

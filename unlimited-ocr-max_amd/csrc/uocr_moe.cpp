@@ -1394,14 +1394,13 @@ int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden, co
   sdn.part_stride = T * H;
   const bool staged = vec && aligned16(ws);
   if (gemm_staged_ok(gu, staged) && gemm_staged_ok(dn, staged)) {
-    e = launch_moe_layer(gu, sgu, dn, sdn, d.g.ctl, spin_limit(kPrefillSpin), s);
+    e = launch_moe_layer(gu, sgu, dn, sdn, d.g.ctl, spin_limit(kPrefillSpin), d.wts, (int)R, s);
   } else {
     e = launch_gemm_phase(gu, sgu, staged, d.g.ctl, s);
     if (e == hipSuccess) e = launch_gemm_phase(dn, sdn, staged, d.g.ctl, s);
   }
   if (e == hipSuccess)
-    e = launch_combine(out, d.y, H, d.wts, d.g.inv, d.sh, (int)T, H, (int)L->top_k, s, sdn.kparts,
-                       d.g.ctl + moe_layer_failed_word());
+    e = launch_combine(out, d.y, H, d.wts, d.g.inv, d.sh, (int)T, H, (int)L->top_k, s, sdn.kparts);
   if (e == hipSuccess && expert_ids) e = hipMemcpyAsync(expert_ids, d.ids, R * sizeof(int32_t), hipMemcpyDeviceToDevice, s);
   if (e == hipSuccess && expert_weights)
     e = hipMemcpyAsync(expert_weights, d.wts, R * sizeof(float), hipMemcpyDeviceToDevice, s);
