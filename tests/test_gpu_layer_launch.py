@@ -21,6 +21,7 @@ SHAPES = {  # experts, hidden, ffn (top 2, 2 shared experts)
     "one": (1, 128, 128),
     "fine gate/up": (8, 1152, 256),  # at int8 group 64: 18 groups a row, down 4
     "fine down": (8, 256, 1152),
+    "wide": (8, 2176, 256),
 }
 
 
@@ -138,7 +139,7 @@ def test_a_wait_without_an_end_is_nan(oracle, monkeypatch, T) -> None:
     assert bits_equal(n(moe(x, workspace=ws)), n(other(x)))
 
 
-@pytest.mark.parametrize("T", [1, 33, 130, 700, 2100])
+@pytest.mark.parametrize("T", [1, 33, 130, 700, 2100, 9000])
 @pytest.mark.parametrize(("shape", "staged"), [("fine gate/up", "gemm_down"), ("fine down", "gemm_gateup")])
 def test_one_phase_staged(oracle, shape, staged, T) -> None:
     """More than 16 int8 groups a row in one phase: only that phase leaves the LDS-staged kernel."""
@@ -150,4 +151,18 @@ def test_one_phase_staged(oracle, shape, staged, T) -> None:
     got = n(moe(x))
     names = [name for name, _ in _lib.timing_end(16)]
     assert staged in names and sum(name.startswith("gemm_") for name in names) == 2
+    assert bits_equal(got, n(other(x)))
+
+
+@pytest.mark.parametrize("T", [2048, 2111, 5000])
+def test_wide_layers_take_two_launches(oracle, T) -> None:
+    """Beyond hidden 2048 each phase has a launch of its own (from 2048 tokens on, the router's limit there)."""
+    from uocr_moe import _lib
+
+    moe, other = _pair(oracle, "wide", False)
+    x = _x(T, SHAPES["wide"][1])
+    _lib.timing_begin(16)
+    got = n(moe(x))
+    names = [name for name, _ in _lib.timing_end(16)]
+    assert [name for name in names if name.startswith("gemm_")] == ["gemm_gateup", "gemm_down"]
     assert bits_equal(got, n(other(x)))

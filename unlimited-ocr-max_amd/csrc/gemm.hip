@@ -1019,12 +1019,12 @@ __device__ __forceinline__ int lds_tile(const GemmProblem& P, const TileRef& t, 
     else
       step_barrier<(LB - LA) * NB + (LA - 1) * NL>();
     if (LA < LB && u + 1 < LB) issue_a(s + LA);
-    if (u + 1 == LB && threadIdx.x == 0) ticket = agent_add(ctl.ticket, 1);
+    if (JOINT && u + 1 == LB && threadIdx.x == 0) ticket = agent_add(ctl.ticket, 1);
     compute(s);
   }
   // every wave has finished reading the stages (and the scales) before the next tile's loads
   step_barrier<0>();
-  if (threadIdx.x == 0) *(int*)lds = ticket;
+  if (JOINT && threadIdx.x == 0) *(int*)lds = ticket;
   if (parts > 1) {
     GemmProblem Q = P;  // range t.e's sums
     Q.outf += t.e * P.part_stride;
@@ -1032,11 +1032,13 @@ __device__ __forceinline__ int lds_tile(const GemmProblem& P, const TileRef& t, 
   } else {
     store_tile<32 * NACT, NPROJ, kGives>(P, t, acc, w, m, h);
   }
-  if constexpr (kGives) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // h is past the L2
-  lds_barrier();
-  ticket = __builtin_amdgcn_readfirstlane(*(const int*)lds);
-  if (kGives && threadIdx.x == 0) (void)agent_add(ctl.done + t.dep * kCtlLine, 1);
-  lds_barrier();
+  if constexpr (JOINT) {
+    if constexpr (kGives) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // h is past the L2
+    lds_barrier();
+    ticket = __builtin_amdgcn_readfirstlane(*(const int*)lds);
+    if (kGives && threadIdx.x == 0) (void)agent_add(ctl.done + t.dep * kCtlLine, 1);
+    lds_barrier();
+  }
   return ticket;
 }
 
@@ -1372,21 +1374,40 @@ __device__ __forceinline__ int broadcast(int v, char* lds) {
   return v;
 }
 
-// One phase of the launch (gate/up, NP = 2, or down, NP = 1) for a workgroup:
-// the tiles of its own XCD's list by ticket, then what is left of the others'.
-// So a workgroup goes on to the down tiles once every gate/up tile has been
-// taken by a running workgroup: a down tile's wait ends whatever else shares
-// the device.  plan(x) prepares XCD x's list and returns its length, run(it,
-// ctl) does tile `it` of it.  STEAL: take other lists' tiles at once, in both
-// phases (many tiles a list: T = 4096 363 -> 350 us).  Otherwise a list's few
-// remaining gate/up tiles are given kPatience polls (some microseconds) to be
-// taken by its own workgroups, which have it planned (taking them at once:
-// T = 291 92 -> 96 us, T = 64 87 -> 93).
+// One phase (gate/up, NP = 2, or down, NP = 1) for a workgroup.  plan(x)
+// prepares XCD x's list and returns its length, run(it, ctl) does tile `it`.
+//
+// JOINT (both phases in the launch): the tiles of its own XCD's list by ticket,
+// then what is left of the others'.  So a workgroup goes on to the down tiles
+// once every gate/up tile has been taken by a running workgroup: a down tile's
+// wait ends whatever else shares the device.  STEAL: take other lists' tiles at
+// once, in both phases (many tiles a list: T = 4096 363 -> 350 us).  Otherwise a
+// list's few remaining gate/up tiles are given kPatience polls (some
+// microseconds) to be taken by its own workgroups, which have it planned (taking
+// them at once: T = 291 92 -> 96 us, T = 64 87 -> 93).
+//
+// Alone: workgroup j of the XCD takes tiles j, j + J, ... of its list, and of a
+// list of at most two rounds the second in reverse, so that the workgroups with
+// the costliest first tiles take the cheapest second ones.  Nothing waits, so no
+// ticket is needed, and the workgroups of an XCD start on different CUs, then a
+// second one on each, where tickets may run a few tiles two to a CU (int8 group
+// 64, T = 4 / 16 71 / 107 us by ticket, 66 / 103 so) and drift apart over many
+// rounds, which then share fewer of a list's operands (bf16, hidden 3072, T =
+// 4096 1690 us by ticket, 1520 so).
 constexpr int kPatience = 16;
 template <int NP, bool STEAL, bool JOINT, typename PlanFn, typename RunFn>
 __device__ __forceinline__ void walk(int32_t* ctl, const Guard& guard, char* lds, PlanFn&& plan, RunFn&& run) {
-  int32_t* lists = ctl + (NP == 2 ? 0 : kXcds) * kCtlLine;
   const int own = (int)blockIdx.x % kXcds;
+  if constexpr (!JOINT) {
+    const int j = (int)blockIdx.x / kXcds, J = (int)gridDim.x / kXcds;
+    const int n = plan(own);
+    for (int k = 0; k * J < n; ++k) {
+      const int it = n <= 2 * J && k == 1 ? 2 * J - 1 - j : j + k * J;
+      if (it < n) (void)run(it, PhaseCtl{});
+    }
+    return;
+  }
+  int32_t* lists = ctl + (NP == 2 ? 0 : kXcds) * kCtlLine;
   uint32_t unseen = (1u << kXcds) - 1;  // lists this workgroup has not run to their end
   for (int x = own;;) {
     const PhaseCtl pc{lists + x * kCtlLine, ctl + kCtlDone, guard};
@@ -1397,7 +1418,7 @@ __device__ __forceinline__ void walk(int32_t* ctl, const Guard& guard, char* lds
     if (it == 0 && threadIdx.x == 0)
       __hip_atomic_store(pc.ticket + 1, n + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     while ((uint32_t)it < (uint32_t)n) it = run(it, pc);  // (an overwritten counter may give any value)
-    if (!STEAL && !(JOINT && NP == 2)) return;
+    if (!STEAL && NP == 1) return;
     unseen &= ~(1u << x);
     if (threadIdx.x < kWave) {
       // a bit per list whose tickets have not run past its length, or whose length is not known yet
@@ -1545,12 +1566,12 @@ __global__ void __launch_bounds__(kGThreads, kWgPerCu) k_moe_layer(GemmProblem a
 
 // One phase alone, the other in a launch of its own.
 template <WKind W0, int NP, bool BAL>
-__global__ void __launch_bounds__(kGThreads, kWgPerCu) k_moe_phase(GemmProblem a, GemmProblem b, int32_t* ctl) {
+__global__ void __launch_bounds__(kGThreads, kWgPerCu) k_moe_phase(GemmProblem a, GemmProblem b) {
   extern __shared__ __attribute__((aligned(16))) char lds_stages[];
   if constexpr (BAL)
-    walk_balanced<W0, NP, false>(a, b, 0, 0, ctl, Guard{}, lds_stages);
+    walk_balanced<W0, NP, false>(a, b, 0, 0, nullptr, Guard{}, lds_stages);
   else
-    walk_classes<W0, NP, false>(a, b, 0, 0, ctl, Guard{}, lds_stages);
+    walk_classes<W0, NP, false>(a, b, 0, 0, nullptr, Guard{}, lds_stages);
 }
 
 // Workgroups of the layer's grid: every CU's resident share, a whole number
@@ -1596,8 +1617,7 @@ bool balanced(const GemmProblem& routed, const GemmProblem& shared, int grid) {
 }
 
 template <WKind W0>
-hipError_t launch_phase(const GemmProblem& routed, const GemmProblem& shared, const char* name, int32_t* ctl,
-                        hipStream_t s) {
+hipError_t launch_phase(const GemmProblem& routed, const GemmProblem& shared, const char* name, hipStream_t s) {
   constexpr size_t lds = kLdsBytes<W0>;
   int grid = 0;
   const hipError_t e = moe_layer_grid<W0>(&grid);
@@ -1605,14 +1625,14 @@ hipError_t launch_phase(const GemmProblem& routed, const GemmProblem& shared, co
   const dim3 g(grid), b(kGThreads);
   if (routed.swiglu) {
     if (balanced<W0>(routed, shared, grid))
-      UOCR_LAUNCH(name, (k_moe_phase<W0, 2, true>), g, b, lds, s, routed, shared, ctl);
+      UOCR_LAUNCH(name, (k_moe_phase<W0, 2, true>), g, b, lds, s, routed, shared);
     else
-      UOCR_LAUNCH(name, (k_moe_phase<W0, 2, false>), g, b, lds, s, routed, shared, ctl);
+      UOCR_LAUNCH(name, (k_moe_phase<W0, 2, false>), g, b, lds, s, routed, shared);
   } else {
     if (balanced<W0>(routed, shared, grid))
-      UOCR_LAUNCH(name, (k_moe_phase<W0, 1, true>), g, b, lds, s, routed, shared, ctl);
+      UOCR_LAUNCH(name, (k_moe_phase<W0, 1, true>), g, b, lds, s, routed, shared);
     else
-      UOCR_LAUNCH(name, (k_moe_phase<W0, 1, false>), g, b, lds, s, routed, shared, ctl);
+      UOCR_LAUNCH(name, (k_moe_phase<W0, 1, false>), g, b, lds, s, routed, shared);
   }
   return hipGetLastError();
 }
@@ -1711,8 +1731,7 @@ static hipError_t launch_fragment(const GemmProblem& routed, const GemmProblem& 
                        : launch_moe_gemm<64, W0, 1, false>(routed, shared, s, name);
 }
 
-hipError_t launch_gemm_phase(const GemmProblem& routed, const GemmProblem& shared, bool vec, int32_t* ctl,
-                             hipStream_t s) {
+hipError_t launch_gemm_phase(const GemmProblem& routed, const GemmProblem& shared, bool vec, hipStream_t s) {
   if (!gemm_shapes_ok(routed, shared)) return hipErrorInvalidValue;
   const bool int8 = routed.kind == kInt8Rows;
   if (!gemm_staged_ok(routed, vec)) {  // 64-row tiles
@@ -1721,8 +1740,8 @@ hipError_t launch_gemm_phase(const GemmProblem& routed, const GemmProblem& share
                 : launch_fragment<kBf16Rows>(routed, shared, name, s);
   }
   const char* name = routed.swiglu ? "gemm_gateup" : "gemm_down";
-  return int8 ? launch_phase<kInt8Rows>(routed, shared, name, ctl, s)
-              : launch_phase<kBf16Rows>(routed, shared, name, ctl, s);
+  return int8 ? launch_phase<kInt8Rows>(routed, shared, name, s)
+              : launch_phase<kBf16Rows>(routed, shared, name, s);
 }
 
 }  // namespace uocr

@@ -201,20 +201,19 @@ struct GemmProblem {
 // multiple of 64); a routed problem has at most 64 groups.
 //
 // gemm_staged_ok: the LDS-staged kernels take the problem (vec: every operand is
-// 16-byte aligned).  ctl: moe_layer_ctl_words(tokens) words, zero before a
-// layer's first launch (the grouping's launch clears them).
+// 16-byte aligned).
 bool gemm_staged_ok(const GemmProblem& routed, bool vec);
-int moe_layer_ctl_words(int64_t tokens);
 // Gate/up and down of a layer in one launch, both staged: dn and sdn read what
-// gu and sgu write.  A down tile waits for its rows at most spin_limit polls,
-// then the launch goes on and the nwts weights of the
+// gu and sgu write.  ctl: moe_layer_ctl_words(tokens) words, zero before the
+// launch (the grouping's launch clears them).  A down tile waits for its rows at
+// most spin_limit polls, then the launch goes on and the nwts weights of the
 // combine, wts, become NaN.
+int moe_layer_ctl_words(int64_t tokens);
 hipError_t launch_moe_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn,
                             const GemmProblem& sdn, int32_t* ctl, uint32_t spin_limit, float* wts, int nwts,
                             hipStream_t s);
 // One phase, staged or with weights at any alignment, with the same bits.
-hipError_t launch_gemm_phase(const GemmProblem& routed, const GemmProblem& shared, bool vec, int32_t* ctl,
-                             hipStream_t s);
+hipError_t launch_gemm_phase(const GemmProblem& routed, const GemmProblem& shared, bool vec, hipStream_t s);
 // The K ranges to cut the shared problem into for this pair (1 or 2).
 int gemm_shared_parts(const GemmProblem& routed, const GemmProblem& shared);
 

@@ -1392,12 +1392,15 @@ int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden, co
   // launch's longest at T = 512 (down 43 -> 35 us).
   sdn.kparts = gemm_shared_parts(dn, sdn);
   sdn.part_stride = T * H;
+  // One launch: its down tiles read h past the L2, once for each of hidden / 256 column tiles.  Up to 8 that
+  // costs less than a second launch (bf16, T = 4096, hidden 1280 / 2048: 421 / 997 us against 434 / 1003),
+  // beyond it costs more (hidden 3072 / 4096, ffn 1408: 1727 / 2265 against 1520 / 2037).
   const bool staged = vec && aligned16(ws);
-  if (gemm_staged_ok(gu, staged) && gemm_staged_ok(dn, staged)) {
+  if (H <= 2048 && gemm_staged_ok(gu, staged) && gemm_staged_ok(dn, staged)) {
     e = launch_moe_layer(gu, sgu, dn, sdn, d.g.ctl, spin_limit(kPrefillSpin), d.wts, (int)R, s);
   } else {
-    e = launch_gemm_phase(gu, sgu, staged, d.g.ctl, s);
-    if (e == hipSuccess) e = launch_gemm_phase(dn, sdn, staged, d.g.ctl, s);
+    e = launch_gemm_phase(gu, sgu, staged, s);
+    if (e == hipSuccess) e = launch_gemm_phase(dn, sdn, staged, s);
   }
   if (e == hipSuccess)
     e = launch_combine(out, d.y, H, d.wts, d.g.inv, d.sh, (int)T, H, (int)L->top_k, s, sdn.kparts);
