@@ -1,11 +1,13 @@
-"""The matrix-instruction GEMVs' host-checkable rules (``csrc/gemv_mfma.hip``), called in the built library.
+"""Host-checkable rules of the matrix-instruction kernels, called in the built library.
 
-``rows_offset`` is the kernel's own lane offset into a wave's 64 weight columns, compiled for the host too.  It
+``rows_offset`` (``csrc/gemv_mfma.hip``) is the kernel's own lane offset into a wave's 64 weight columns, compiled for the host too.  It
 is compared with exact integers over the widths that the ops admit, a matrix of more than 2 GiB among them;
 the 32-bit product of an unclamped column fails the same comparison.
 
 ``rows_routed_ok`` and ``rows_dense_ok`` say which calls these kernels take.  A call without any k is not one of
 them: their loops read at least one step, and a plan of no chunks divides by their number.
+
+``gemm_staged_ok`` (``csrc/gemm.hip``) admits what the prefill's LDS-staged kernels can address and hold.
 """
 
 from __future__ import annotations
@@ -105,3 +107,29 @@ def test_dense_call_without_k_returns() -> None:
             "assert rc != 0 and err.value")
     env = {**os.environ, "PYTHONPATH": str(PKG_DIR), "HIP_VISIBLE_DEVICES": "-1", "ROCR_VISIBLE_DEVICES": "-1"}
     assert subprocess.run([sys.executable, "-c", code], env=env, timeout=300).returncode == 0
+
+
+class _GemmProblem(ctypes.Structure):
+    """``GemmProblem`` of ``csrc/uocr_kernels.h``."""
+
+    _fields_ = [("a", ctypes.c_void_p), ("lda", ctypes.c_int64), ("a_by_token", ctypes.c_int), ("x_div", ctypes.c_int),
+                ("p", _Proj * 2), ("kind", ctypes.c_int), ("N", ctypes.c_int), ("K", ctypes.c_int),
+                ("groups", ctypes.c_int), ("rows", _Rows), ("tile_start", ctypes.c_void_p),
+                ("max_groups", ctypes.c_int), ("M", ctypes.c_int), ("swiglu", ctypes.c_int), ("outb", ctypes.c_void_p),
+                ("outf", ctypes.c_void_p), ("ldo", ctypes.c_int64), ("out_by_position", ctypes.c_int),
+                ("kparts", ctypes.c_int), ("part_stride", ctypes.c_int64)]
+
+
+@pytest.mark.parametrize(("kind", "k", "groups", "max_groups", "vec", "takes"), [
+    (INT8_ROWS, 1280, 10, 64, True, True), (INT8_ROWS, 1280, 10, 64, False, False),
+    (INT8_ROWS, 1024, 16, 1, True, True), (INT8_ROWS, 1088, 17, 1, True, False),
+    (BF16_ROWS, 6848, 1, 64, True, True), (BF16_ROWS, 1280, 1, 65, True, False),
+    # 256 weight rows of a tile within 32 bits
+    (INT8_ROWS, (1 << 24) - 128, 8, 1, True, True), (INT8_ROWS, 1 << 24, 8, 1, True, False),
+    (BF16_ROWS, (1 << 23) - 128, 1, 1, True, True), (BF16_ROWS, 1 << 23, 1, 1, True, False),
+])
+def test_staged_gemm_takes(kind, k, groups, max_groups, vec, takes) -> None:
+    problem = _GemmProblem(kind=kind, N=128, K=k, groups=groups, max_groups=max_groups)
+    check = _internal("_ZN4uocr14gemm_staged_okERKNS_11GemmProblemEb", ctypes.c_bool, ctypes.POINTER(_GemmProblem),
+                      ctypes.c_bool)
+    assert check(ctypes.byref(problem), vec) == takes

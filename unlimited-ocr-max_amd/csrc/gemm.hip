@@ -903,7 +903,7 @@ __device__ __forceinline__ int lds_tile(const GemmProblem& P, const TileRef& t, 
     const int mm = rr & 31;
     const int row = min(NPROJ == 2 ? 32 * w + mm : 64 * w + rr, P.N - 1 - t.n0);
     const int c = (j % (RB / 16)) ^ (W == kInt8Rows ? swz64(rr) : swz(rr));
-    boff[i] = (uint32_t)(row * RB * (P.K / BK) + 16 * c);
+    boff[i] = (uint32_t)row * (uint32_t)(RB * (P.K / BK)) + (uint32_t)(16 * c);
   }
   const int64_t bstep = W == kBf16KBlocked ? (int64_t)(BK / 16) * P.N * 32 : RB;
   const int64_t bfirst = W == kBf16KBlocked ? (int64_t)t.n0 * 32
@@ -1710,9 +1710,12 @@ int moe_layer_ctl_words(int64_t tokens) {
 // lane per routed group in the placement's plan; the fragment-load kernel
 // takes the rest.  Each phase by itself: at int8 group 64, hidden 1280 and ffn
 // 896, gate/up has 20 groups a row and down 14 (T = 512 / 4096 149 / 570 us
-// with both on the fragment-load kernel, 137 / 495 with gate/up alone).
+// with both on the fragment-load kernel, 137 / 495 with gate/up alone).  A
+// weight row is short enough for 32-bit offsets over a tile's 256 rows.
 bool gemm_staged_ok(const GemmProblem& routed, bool vec) {
-  return vec && routed.max_groups <= kWave && (routed.kind != kInt8Rows || routed.groups <= kMaxScaleGroups);
+  const int64_t row_bytes = (int64_t)routed.K * (routed.kind == kInt8Rows ? 1 : 2);
+  return vec && routed.max_groups <= kWave && kWRowsWg * row_bytes <= UINT32_MAX &&
+         (routed.kind != kInt8Rows || routed.groups <= kMaxScaleGroups);
 }
 
 hipError_t launch_moe_layer(const GemmProblem& gu, const GemmProblem& sgu, const GemmProblem& dn,
