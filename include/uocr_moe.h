@@ -308,7 +308,8 @@ int uocr_moe_decode_stack(float* out, const float* x, int64_t rows, int64_t hidd
  * path).  x fp32 [T, H] -> out fp32 [T, H].  The top-k experts of every token
  * run as a grouped GEMM on the bf16 matrix cores: int8 weights dequantised to
  * bf16_rne(f32(q)*scale) (the reference's prefill values), activations
- * rounded to bf16, fp32 accumulation.  H, F, Fs multiples of 128.  Calls that
+ * rounded to bf16, fp32 accumulation.  H, F, Fs multiples of 128; T * H, T * k * F
+ * and T * Fs below 2^31.  Calls that
  * overlap in time must not share a workspace (nor, with workspace == NULL, a
  * stream's own one across captured graphs): their tables, rows and control
  * words overwrite each other.  The one in-kernel wait is bounded (about a

@@ -133,3 +133,12 @@ def test_staged_gemm_takes(kind, k, groups, max_groups, vec, takes) -> None:
     check = _internal("_ZN4uocr14gemm_staged_okERKNS_11GemmProblemEb", ctypes.c_bool, ctypes.POINTER(_GemmProblem),
                       ctypes.c_bool)
     assert check(ctypes.byref(problem), vec) == takes
+
+
+def test_prefill_beyond_its_row_offsets_is_refused() -> None:
+    """h of 400 000 tokens (top 6, ffn 896) has more than 2^31 elements: refused before anything is allocated."""
+    from uocr_moe import _lib
+
+    layer = _lib.Layer(64, 1280, 896, 1792, 6, 128, 1, 0, *[16] * 10)
+    with pytest.raises(_lib.UocrError, match="seq out of range"):
+        _lib.call("uocr_moe_forward", 16, 16, 400_000, 1280, ctypes.byref(layer), None, None, None, 0, None)

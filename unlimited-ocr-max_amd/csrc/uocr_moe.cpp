@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -1297,7 +1298,10 @@ int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden, co
   const bool vec = aligned16(L->gate_proj) && aligned16(L->up_proj) && aligned16(L->down_proj) &&
                    aligned16(L->shared_gate) && aligned16(L->shared_up) && aligned16(L->shared_down);
   if ((reinterpret_cast<uintptr_t>(x) & 3u) != 0) return fail(err, errlen, "%s: x must be 4-byte aligned", op);
-  if (seq < 0 || seq * L->top_k > ((int64_t)1 << 28)) return fail(err, errlen, "%s: seq out of range", op);
+  // the GEMMs' row offsets (elements of x, h and the shared h) are 32-bit
+  const int64_t widest = std::max(std::max(L->hidden, L->top_k * L->ffn), L->shared_ffn);
+  if (seq < 0 || seq * L->top_k > ((int64_t)1 << 28) || seq > INT32_MAX / widest)
+    return fail(err, errlen, "%s: seq out of range", op);
   if (seq == 0) return 0;
   const hipStream_t s = (hipStream_t)stream;
   const int64_t T = seq, R = seq * L->top_k;
