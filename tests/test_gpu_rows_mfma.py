@@ -118,3 +118,28 @@ def test_no_k(rows) -> None:
     ids = torch.arange(rows, dtype=torch.int32, device="cuda:0") % 3
     out = torch.full((rows, 70), float("nan"), device="cuda:0")
     assert not n(ops.moe_bf16_qmv(x, ids, torch.empty((3, 70, 0), dtype=torch.bfloat16, device="cuda:0"), out=out)).any()
+
+
+@pytest.mark.parametrize(("kind", "e", "n_", "rows", "kernel"), [
+    ("int8", 8, 1088, 7, "gemv_op"), ("int8", 8, 1088, 8, "rows_op"), ("int8", 8, 1088, 100, "rows_op"),
+    ("int8", 16, 256, 31, "gemv_op"), ("int8", 16, 256, 32, "rows_op"), ("int8", 3, 320, 200, "gemv_op"),
+    ("bf16", 8, 384, 4, "gemv_op"), ("bf16", 8, 384, 5, "rows_op"),
+    ("bf16", 1, 384, 8, "gemv_op"), ("bf16", 1, 384, 9, "rows_op"),
+])
+def test_routed_ops_at_the_edges_of_the_rule(oracle, kind, e, n_, rows, kernel) -> None:
+    """Few column waves stay on the VALU kernel, a stack of few experts and many rows does not; same bits."""
+    from uocr_moe import _lib, ops
+
+    rng = np.random.default_rng(rows)
+    ids = rng.integers(0, e, rows).astype(np.int32)
+    x = rng.standard_normal((rows, 256)).astype(np.float32)
+    _lib.timing_begin(8)
+    if kind == "int8":
+        w = rng.integers(-127, 128, (e, n_, 256)).astype(np.int8)
+        s = rng.uniform(1e-4, 1e-2, (e, n_, 2)).astype(np.float32)
+        got, want = n(ops.moe_int8_qmv(t(x), t(ids), t(w), t(s))), oracle.moe_int8_qmv(x, ids, w, s)
+    else:
+        w = oracle.bf16_bits(rng.standard_normal((e, n_, 256)).astype(np.float32))
+        got, want = n(ops.moe_bf16_qmv(t(x), t(ids), t(w))), oracle.moe_bf16_qmv_chunked(x, ids, w)
+    assert kernel in [name for name, _ in _lib.timing_end(8)]
+    assert bits_equal(got, want)

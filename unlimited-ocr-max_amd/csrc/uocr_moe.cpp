@@ -391,10 +391,18 @@ int routed_qmv(const char* op, WKind kind, float* result, const float* x, const 
   }
   a.batch = batch_for(a.nchunks);
   a.rows = rows_of(g);
-  // Few int8 groups (a token or two) leave most SIMDs without a wave of the matrix path, whose waves take
-  // all chunks of their columns: 6 rows of 64 experts' gate took 16.1 us there and 7.8 us with a wave per
-  // chunk; 18 rows 16.7 against 22.2 us.
-  e = rows_routed_ok(a) && (kind != kInt8Rows || max_groups > 8) ? launch_rows_routed(a, max_groups, s) : launch_gemv(a, max_groups, 1, waves_for(a.batch), s);
+  // A wave of the matrix path takes all chunks of its 64 columns, so few groups of narrow outputs leave most
+  // SIMDs idle, where the VALU kernel has a wave per chunk but goes over a group's rows eight at a time, with
+  // more work for each.  Both measured with cold weights, us (VALU, matrix), `waves` in brackets: int8, 64
+  // experts N = 896, K = 1280, 4 rows (56) 20.9, 21.2, 9 rows (126) 23.4, 21.8; N = 1280, K = 896, 6 rows (120)
+  // 17.1, 17.8; 16 experts N = 256, 16 rows (64) 11.3, 12.5, 96 rows 15.3, 14.0; 8 experts N = 2048, K = 4096, 8
+  // rows (256) 89, 49.  bf16, 64 experts N = 896, 1 row (14) 22.0, 23.5, 2 rows (28) 25.0, 24.6; 1 expert, 8 rows
+  // (14) 24.8, 26.4, 12 rows 40, 32; 64 experts N = 2048, K = 2048, 2 rows (64) 32.6, 34.4, 5 rows (160) 36.7, 35.6.
+  const int64_t waves = (int64_t)max_groups * ((N + 63) / 64);
+  const bool fills = kind == kInt8Rows ? waves > 120 || (waves >= 64 && k >= 2 * max_groups)
+                                       : waves > (K >= 2048 ? 64 : 24) || k > 8 * max_groups;
+  e = fills && rows_routed_ok(a) ? launch_rows_routed(a, max_groups, s)
+                                 : launch_gemv(a, max_groups, 1, waves_for(a.batch), s);
   return e == hipSuccess ? 0 : hip_fail(err, errlen, op, e);
 }
 
