@@ -658,8 +658,7 @@ def prefill_gemm_dispatches(rows: list) -> dict[str, list]:
     over the 11 layers, then T=4096 and the adversarial T=4096 over 4 layers each."""
     gemms = [r for r in rows if "k_moe_layer" in r[1]]
     n512, n4k = LAYERS, PREFILL_4K_LAYERS
-    return {"t512_gemm": gemms[:n512], "t4096_gemm": gemms[n512:n512 + n4k],
-            "t4096_adversarial_gemm": gemms[n512 + n4k:]}
+    return {"t512": gemms[:n512], "t4096": gemms[n512:n512 + n4k], "t4096_adversarial": gemms[n512 + n4k:]}
 
 
 def prefill_probe() -> int:
@@ -830,20 +829,17 @@ def main() -> int:
             results["prefill_counters"] = pc
             for key, label in (("prefill_int8_t512", "t512"), ("prefill_int8_t4096", "t4096"),
                                ("prefill_int8_t4096_adversarial", "t4096_adversarial")):
-                r = results.get(key)
-                if r is None:
+                r, c = results.get(key), pc.get(label)
+                if r is None or c is None:
                     continue
-                for kind, kname in (("gemm", "gemm_layer"),):
-                    c = pc.get(f"{label}_{kind}")
-                    us = r["kernels_us_avg"].get(kname)
-                    if c is None or us is None:
-                        continue
-                    c["kernel_us"] = us
-                    c["mfma_tflops_executed"] = round(c["mfma_flops_per_launch"] / (us * 1e-6) / 1e12, 1)
-                    if "traffic_bytes" in c:
-                        c["traffic_gbs"] = round(c["traffic_bytes"] / (us * 1e-6) / 1e9, 1)
-                r["mfma_busy_frac"] = {k: pc[f"{label}_{k}"]["mfma_busy_frac"] for k in ("gemm",)
-                                       if f"{label}_{k}" in pc}
+                r["mfma_busy_frac"] = c["mfma_busy_frac"]
+                us = r["kernels_us_avg"].get("gemm_layer")
+                if us is None:
+                    continue
+                c["kernel_us"] = us
+                c["mfma_tflops_executed"] = round(c["mfma_flops_per_launch"] / (us * 1e-6) / 1e12, 1)
+                if "traffic_bytes" in c:
+                    c["traffic_gbs"] = round(c["traffic_bytes"] / (us * 1e-6) / 1e9, 1)
     line = {
         "metric": METRIC,
         "value": b1["us_per_layer"],

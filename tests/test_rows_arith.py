@@ -114,10 +114,9 @@ class _GemmProblem(ctypes.Structure):
 
     _fields_ = [("a", ctypes.c_void_p), ("lda", ctypes.c_int64), ("a_by_token", ctypes.c_int), ("x_div", ctypes.c_int),
                 ("p", _Proj * 2), ("kind", ctypes.c_int), ("N", ctypes.c_int), ("K", ctypes.c_int),
-                ("groups", ctypes.c_int), ("rows", _Rows), ("tile_start", ctypes.c_void_p),
-                ("max_groups", ctypes.c_int), ("M", ctypes.c_int), ("swiglu", ctypes.c_int), ("outb", ctypes.c_void_p),
-                ("outf", ctypes.c_void_p), ("ldo", ctypes.c_int64), ("out_by_position", ctypes.c_int),
-                ("kparts", ctypes.c_int), ("part_stride", ctypes.c_int64)]
+                ("groups", ctypes.c_int), ("rows", _Rows), ("max_groups", ctypes.c_int), ("M", ctypes.c_int),
+                ("swiglu", ctypes.c_int), ("outb", ctypes.c_void_p), ("outf", ctypes.c_void_p), ("ldo", ctypes.c_int64),
+                ("out_by_position", ctypes.c_int), ("kparts", ctypes.c_int), ("part_stride", ctypes.c_int64)]
 
 
 @pytest.mark.parametrize(("kind", "k", "groups", "max_groups", "vec", "takes"), [

@@ -250,11 +250,6 @@ __device__ __forceinline__ i32x4 ld16_any(const char* p) {
   __builtin_memcpy(&v, (const UOCR_GLOBAL char*)p, 16);
   return v;
 }
-template <bool VEC>
-__device__ __forceinline__ i32x4 ld16w(const char* p) {
-  if constexpr (VEC) return *(const UOCR_GLOBAL i32x4*)p;
-  else return ld16_any(p);
-}
 
 // One K step of one wave's weights, per lane: the 32 k of the lane's column
 // in each block (16-byte pieces), and for int8 the step's scale of each.
@@ -301,19 +296,19 @@ __device__ __forceinline__ WCursor wcursor(const GemmProblem& P, const TileRef& 
   return c;
 }
 
-template <WKind W, bool VEC>
+template <WKind W>
 __device__ __forceinline__ void load_w(const WCursor& c, int k, WStep<W>& o) {
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
     const char* q = c.p[b] + (int64_t)k * c.step;
     if constexpr (W == kBf16KBlocked) {
-      o.v[b][0] = ld16w<VEC>(q);
-      o.v[b][1] = ld16w<VEC>(q + 16);
-      o.v[b][2] = ld16w<VEC>(q + c.kblock);
-      o.v[b][3] = ld16w<VEC>(q + c.kblock + 16);
+      o.v[b][0] = ld16_any(q);
+      o.v[b][1] = ld16_any(q + 16);
+      o.v[b][2] = ld16_any(q + c.kblock);
+      o.v[b][3] = ld16_any(q + c.kblock + 16);
     } else {
 #pragma unroll
-      for (int i = 0; i < WStep<W>::kPieces; ++i) o.v[b][i] = ld16w<VEC>(q + 16 * i);
+      for (int i = 0; i < WStep<W>::kPieces; ++i) o.v[b][i] = ld16_any(q + 16 * i);
     }
     if constexpr (W == kInt8Rows) {
       // the step lies in group k / (steps per group); k < 2^16, so the float
@@ -412,13 +407,13 @@ struct Pipe {
 // loads issued NS - 1 or more steps earlier.  The loads' step index is
 // clamped to the last step (re-reading it is harmless), so the loop body has
 // no branches and the compiler's waits stay exact.
-template <int u, int BM, WKind W, bool VEC>
+template <int u, int BM, WKind W>
 __device__ __forceinline__ void pipe_step(Pipe<BM, W>& p, const GemmProblem& P, const int (&aoff)[BM / 32],
                                           const WCursor& cur, uint16_t* lds, int s, int S, int m, int h) {
   constexpr int NS = Pipe<BM, W>::NS;
   load_a<BM>(P.a, aoff, min(s + NS, S - 1), p.as[u % NS]);  // as[u % NS] held step s, already in LDS
   mfma_step<BM, W>(p.acc, lds + (u & 1) * BM * BK, p.ws[u % NS], m, h);
-  load_w<W, VEC>(cur, min(s + NS, S - 1), p.ws[u % NS]);
+  load_w<W>(cur, min(s + NS, S - 1), p.ws[u % NS]);
   // the other buffer was last read in step s - 1, before the barrier that ended it
   store_a<BM>(p.as[(u + 1) % NS], lds + ((u + 1) & 1) * BM * BK);
   lds_barrier();
@@ -512,7 +507,7 @@ __device__ __forceinline__ void store_tile(const GemmProblem& P, const TileRef& 
   }
 }
 
-template <int BM, WKind W, int NPROJ, bool VEC>
+template <int BM, WKind W, int NPROJ>
 __device__ void gemm_tile(const GemmProblem& P, const TileRef& t, uint16_t* lds) {
   constexpr int MB = BM / 32;
   constexpr int NS = kWStages<W>;
@@ -540,7 +535,7 @@ __device__ void gemm_tile(const GemmProblem& P, const TileRef& t, uint16_t* lds)
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
     load_a<BM>(P.a, aoff, min(i, S - 1), p.as[i]);
-    load_w<W, VEC>(cur, min(i, S - 1), p.ws[i]);
+    load_w<W>(cur, min(i, S - 1), p.ws[i]);
   }
   store_a<BM>(p.as[0], lds);
   lds_barrier();
@@ -549,11 +544,11 @@ __device__ void gemm_tile(const GemmProblem& P, const TileRef& t, uint16_t* lds)
   const int rounds = S / NS;
   for (int rd = 0; rd < rounds; ++rd) {
     const int s = rd * NS;
-    pipe_step<0, BM, W, VEC>(p, P, aoff, cur, lds, s, S, m, h);
-    pipe_step<1, BM, W, VEC>(p, P, aoff, cur, lds, s + 1, S, m, h);
+    pipe_step<0, BM, W>(p, P, aoff, cur, lds, s, S, m, h);
+    pipe_step<1, BM, W>(p, P, aoff, cur, lds, s + 1, S, m, h);
     if constexpr (NS == 4) {
-      pipe_step<2, BM, W, VEC>(p, P, aoff, cur, lds, s + 2, S, m, h);
-      pipe_step<3, BM, W, VEC>(p, P, aoff, cur, lds, s + 3, S, m, h);
+      pipe_step<2, BM, W>(p, P, aoff, cur, lds, s + 2, S, m, h);
+      pipe_step<3, BM, W>(p, P, aoff, cur, lds, s + 3, S, m, h);
     }
   }
   if (NS == 4 && rounds * NS < S) {
@@ -570,9 +565,11 @@ __device__ void gemm_tile(const GemmProblem& P, const TileRef& t, uint16_t* lds)
 // The routed problem `a` (weights W0) and the shared experts' `b` (K-blocked
 // bf16) in one persistent launch: each XCD's workgroups walk that XCD's tiles
 // of a, then of b.
-template <int BM, WKind W0, int NP, bool VEC>
+constexpr int kFragmentBM = 64;  // rows per tile
+template <WKind W0, int NP>
 __global__ void __launch_bounds__(kGThreads) k_moe_gemm(GemmProblem a, GemmProblem b) {
   extern __shared__ uint16_t lds[];
+  constexpr int BM = kFragmentBM;
   constexpr int bn = kWRowsWg / NP;
   const int x = (int)blockIdx.x % kXcds;
   const int j = (int)blockIdx.x / kXcds;
@@ -585,17 +582,18 @@ __global__ void __launch_bounds__(kGThreads) k_moe_gemm(GemmProblem a, GemmProbl
   const int nb = __builtin_amdgcn_readlane(fb, kWave - 1);
   for (int it = j; it < na + nb; it += J) {
     if (it < na) {
-      gemm_tile<BM, W0, NP, VEC>(a, tile_at<BM>(a, pa, x, fa, it, bn), lds);
+      gemm_tile<BM, W0, NP>(a, tile_at<BM>(a, pa, x, fa, it, bn), lds);
     } else {
       const TileRef t = tile_at<BM>(b, pb, x, fb, it - na, bn);
-      for (int r = 0; r < parts_of(b); ++r) gemm_tile<BM, kBf16KBlocked, NP, VEC>(part_problem(b, r), t, lds);
+      for (int r = 0; r < parts_of(b); ++r) gemm_tile<BM, kBf16KBlocked, NP>(part_problem(b, r), t, lds);
     }
   }
 }
 
 // Workgroups of the persistent grid: every CU's resident share, a whole
 // number per XCD.
-template <int BM, WKind W0, int NP, bool VEC>
+constexpr size_t kFragmentLds = (size_t)2 * kFragmentBM * BK * sizeof(uint16_t);
+template <WKind W0, int NP>
 hipError_t moe_gemm_grid(int* grid) {
   static std::atomic<int> cached{0};
   int g = cached.load(std::memory_order_relaxed);
@@ -604,8 +602,7 @@ hipError_t moe_gemm_grid(int* grid) {
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e == hipSuccess)
-      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_moe_gemm<BM, W0, NP, VEC>, kGThreads,
-                                                       (size_t)2 * BM * BK * sizeof(uint16_t));
+      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_moe_gemm<W0, NP>, kGThreads, kFragmentLds);
     if (e != hipSuccess) return e;
     g = (cus / kXcds > 0 ? cus / kXcds : 1) * (per_cu > 0 ? per_cu : 1) * kXcds;
     cached.store(g, std::memory_order_relaxed);
@@ -614,13 +611,12 @@ hipError_t moe_gemm_grid(int* grid) {
   return hipSuccess;
 }
 
-template <int BM, WKind W0, int NP, bool VEC = true>
+template <WKind W0, int NP>
 hipError_t launch_moe_gemm(const GemmProblem& routed, const GemmProblem& shared, hipStream_t s, const char* name) {
   int grid = 0;
-  const hipError_t e = moe_gemm_grid<BM, W0, NP, VEC>(&grid);
+  const hipError_t e = moe_gemm_grid<W0, NP>(&grid);
   if (e != hipSuccess) return e;
-  UOCR_LAUNCH(name, (k_moe_gemm<BM, W0, NP, VEC>), dim3(grid), dim3(kGThreads), (size_t)2 * BM * BK * sizeof(uint16_t),
-              s, routed, shared);
+  UOCR_LAUNCH(name, (k_moe_gemm<W0, NP>), dim3(grid), dim3(kGThreads), kFragmentLds, s, routed, shared);
   return hipGetLastError();
 }
 
@@ -1730,14 +1726,14 @@ hipError_t launch_moe_layer(const GemmProblem& gu, const GemmProblem& sgu, const
 template <WKind W0>
 static hipError_t launch_fragment(const GemmProblem& routed, const GemmProblem& shared, const char* name,
                                   hipStream_t s) {
-  return routed.swiglu ? launch_moe_gemm<64, W0, 2, false>(routed, shared, s, name)
-                       : launch_moe_gemm<64, W0, 1, false>(routed, shared, s, name);
+  return routed.swiglu ? launch_moe_gemm<W0, 2>(routed, shared, s, name)
+                       : launch_moe_gemm<W0, 1>(routed, shared, s, name);
 }
 
 hipError_t launch_gemm_phase(const GemmProblem& routed, const GemmProblem& shared, bool vec, hipStream_t s) {
   if (!gemm_shapes_ok(routed, shared)) return hipErrorInvalidValue;
   const bool int8 = routed.kind == kInt8Rows;
-  if (!gemm_staged_ok(routed, vec)) {  // 64-row tiles
+  if (!gemm_staged_ok(routed, vec)) {
     const char* name = routed.swiglu ? "gemm_gateup_any" : "gemm_down_any";
     return int8 ? launch_fragment<kInt8Rows>(routed, shared, name, s)
                 : launch_fragment<kBf16Rows>(routed, shared, name, s);

@@ -435,7 +435,7 @@ __device__ __forceinline__ uint64_t same_key_lanes(int key, int bits) {
 
 // Groups R rows by clamped expert id, stably: a group holds its rows in row
 // order.  `idof(r)` returns row r's raw id.  One workgroup of up to 16 waves
-// and E <= blockDim.x; `hist` is LDS of (waves x E) ints, `part` of 3 x 16.
+// and E <= blockDim.x; `hist` is LDS of (waves x E) ints, `part` of 2 x 16.
 //
 // Wave w owns the rows [w * chunk, (w + 1) * chunk).  Pass 1 counts its rows
 // per expert, 64 rows at a time: the lanes holding one expert find each other
@@ -445,7 +445,7 @@ __device__ __forceinline__ uint64_t same_key_lanes(int key, int bits) {
 // again, placing each at its wave's cursor plus its rank among the batch's
 // lanes of the same expert.  No atomics, and the order is fixed.
 template <typename IdOf>
-__device__ void group_rows(IdOf idof, int R, int E, int bm, const GroupTables& g, int* hist, int* part) {
+__device__ void group_rows(IdOf idof, int R, int E, const GroupTables& g, int* hist, int* part) {
   const int tid = (int)threadIdx.x;
   const int nt = (int)blockDim.x;
   const int nw = nt / kWave;
@@ -465,7 +465,7 @@ __device__ void group_rows(IdOf idof, int R, int E, int bm, const GroupTables& g
   }
   __syncthreads();
 
-  // per expert: rows, row tiles and whether it is a group; exclusive prefix
+  // per expert: rows and whether it is a group; exclusive prefix
   // sums over the experts (per wave, then across the waves' totals)
   int c = 0;
   if (tid < E) {
@@ -475,32 +475,27 @@ __device__ void group_rows(IdOf idof, int R, int E, int bm, const GroupTables& g
       c += h;
     }
   }
-  const int tiles = c > 0 ? (c + bm - 1) / bm : 0;
   const int nz = c > 0 ? 1 : 0;
-  const int ic = wave_scan_i(c), it = wave_scan_i(tiles), in = wave_scan_i(nz);
+  const int ic = wave_scan_i(c), in = wave_scan_i(nz);
   if (lane_id() == kWave - 1) {
     part[w] = ic;
-    part[16 + w] = it;
-    part[32 + w] = in;
+    part[16 + w] = in;
   }
   __syncthreads();
-  int pc = 0, pt = 0, pn = 0;
+  int pc = 0, pn = 0;
   for (int v = 0; v < w; ++v) {
     pc += part[v];
-    pt += part[16 + v];
-    pn += part[32 + v];
+    pn += part[16 + v];
   }
-  const int start = pc + ic - c, tile0 = pt + it - tiles, grp = pn + in - nz;
+  const int start = pc + ic - c, grp = pn + in - nz;
   if (tid < E) {
     if (c > 0) {
       stg(g.group_expert + grp, tid);
       stg(g.group_start + grp, start);
-      if (g.tile_start) stg(g.tile_start + grp, tile0);
     }
     for (int v = 0; v < nw; ++v) hist[v * E + tid] += start;
     if (tid == E - 1) {
       stg(g.group_start + grp + nz, start + c);
-      if (g.tile_start) stg(g.tile_start + grp + nz, tile0 + tiles);
       stg(g.n_groups, grp + nz);
     }
   }
@@ -523,12 +518,12 @@ __device__ void group_rows(IdOf idof, int R, int E, int bm, const GroupTables& g
 
 // LDS of group_rows for a workgroup of `threads` threads.
 __host__ __device__ constexpr size_t group_lds_bytes(int threads, int E) {
-  return ((size_t)(threads / 64) * E + 48) * sizeof(int);
+  return ((size_t)(threads / 64) * E + 32) * sizeof(int);
 }
 
-__global__ void __launch_bounds__(1024) k_group(const int32_t* __restrict__ ids, int R, int E, int bm, GroupTables g) {
+__global__ void __launch_bounds__(1024) k_group(const int32_t* __restrict__ ids, int R, int E, GroupTables g) {
   extern __shared__ int lds_group[];
-  group_rows([&](int r) { return ids[r]; }, R, E, bm, g, lds_group + 48, lds_group);
+  group_rows([&](int r) { return ids[r]; }, R, E, g, lds_group + 32, lds_group);
 }
 
 // ---------------------------------------------------------------- prefill routing over many workgroups
@@ -716,7 +711,7 @@ __global__ void __launch_bounds__(kRouteWaves * 64) k_logits_topk(
 constexpr int kScatterRows = 256;  // rows ranked at once (a pass per 256 rows of a block)
 
 __global__ void __launch_bounds__(256) k_group_scatter_hist(const int32_t* __restrict__ ids, int T, int E, int topk,
-                                                            int bm, int blocks, int block_tokens,
+                                                            int blocks, int block_tokens,
                                                             const int32_t* __restrict__ hist, GroupTables g) {
   __shared__ int part_before[4][64];
   __shared__ int wcnt[4][64];  // a pass's rows per (wave, expert)
@@ -753,21 +748,18 @@ __global__ void __launch_bounds__(256) k_group_scatter_hist(const int32_t* __res
     // per-expert sums (in a fixed order), then the scans over the experts in one wave
     before = part_before[0][e] + part_before[1][e] + part_before[2][e] + part_before[3][e];
     tot = e < E ? part_tot[0][e] + part_tot[1][e] + part_tot[2][e] + part_tot[3][e] : 0;
-    const int tiles = tot > 0 ? (tot + bm - 1) / bm : 0;
     const int nz = tot > 0 ? 1 : 0;
-    const int ic = wave_scan_i(tot), it = wave_scan_i(tiles), in = wave_scan_i(nz);
-    const int start = ic - tot, tile0 = it - tiles, grp = in - nz;
+    const int ic = wave_scan_i(tot), in = wave_scan_i(nz);
+    const int start = ic - tot, grp = in - nz;
     if (e < E) {
       cursor[e] = start + before;
       if (b == 0) {
         if (tot > 0) {
           stg(g.group_expert + grp, e);
           stg(g.group_start + grp, start);
-          if (g.tile_start) stg(g.tile_start + grp, tile0);
         }
         if (e == E - 1) {
           stg(g.group_start + grp + nz, start + tot);
-          if (g.tile_start) stg(g.tile_start + grp + nz, tile0 + tiles);
           stg(g.n_groups, grp + nz);
         }
       }
@@ -817,7 +809,7 @@ __global__ void __launch_bounds__(1024) k_route_small(const float* __restrict__ 
                scratch[threadIdx.x >> 6]);
   }
   __syncthreads();
-  group_rows([&](int r) { return ids_lds[r]; }, T * topk, E, 1, g, lds_group + 48, lds_group);
+  group_rows([&](int r) { return ids_lds[r]; }, T * topk, E, g, lds_group + 32, lds_group);
 }
 
 // ---------------------------------------------------------------- combine
@@ -872,7 +864,7 @@ __global__ void __launch_bounds__(kCombineThreads) k_combine(float* __restrict__
 hipError_t launch_logits(float* logits, const float* x, int64_t ldx, const float* router, int T, int E, int H,
                          uint16_t* xb, hipStream_t s, int32_t* zero, int nzero) {
   if (T <= 0) return hipSuccess;
-  if (H == 20 * kWave && E == 64 && T >= kRingTokens) {
+  if (ring_router(T, E, H)) {
     // every XCD an equal share of the token blocks (those past T return at once)
     const int ntb = (T + 31) / 32;
     const dim3 grid((unsigned)(kXcds * ((ntb + kXcds - 1) / kXcds) * ((E + 15) / 16)));
@@ -922,22 +914,22 @@ hipError_t launch_softmax_topk(const float* logits, int T, int E, int topk, int 
   return hipGetLastError();
 }
 
-hipError_t launch_group(const int32_t* ids, int R, int E, int bm, const GroupTables& g, hipStream_t s) {
+hipError_t launch_group(const int32_t* ids, int R, int E, const GroupTables& g, hipStream_t s) {
   if (E > kMaxGroupExperts) return hipErrorInvalidValue;
-  UOCR_LAUNCH("group", k_group, dim3(1), dim3(1024), group_lds_bytes(1024, E), s, ids, R, E, bm, g);
+  UOCR_LAUNCH("group", k_group, dim3(1), dim3(1024), group_lds_bytes(1024, E), s, ids, R, E, g);
   return hipGetLastError();
 }
 
 int route_count_blocks(int T) { return (T + kCountTokens - 1) / kCountTokens; }
 
 hipError_t launch_topk_group(const float* logits, int T, int E, int topk, int renorm, int32_t* ids32, float* wts,
-                             int bm, const GroupTables& g, int32_t* hist, hipStream_t s) {
+                             const GroupTables& g, int32_t* hist, hipStream_t s) {
   if (T <= 0) return hipSuccess;
   if (E > kRouteMaxExperts) return hipErrorInvalidValue;
   const int blocks = route_count_blocks(T);
   UOCR_LAUNCH("topk_count", k_topk_count, dim3(blocks), dim3(kCountThreads), 0, s, logits, T, E, topk, renorm, ids32,
               wts, hist);
-  UOCR_LAUNCH("group_scatter", k_group_scatter_hist, dim3(blocks), dim3(256), 0, s, ids32, T, E, topk, bm, blocks,
+  UOCR_LAUNCH("group_scatter", k_group_scatter_hist, dim3(blocks), dim3(256), 0, s, ids32, T, E, topk, blocks,
               kCountTokens, hist, g);
   return hipGetLastError();
 }
@@ -959,13 +951,13 @@ hipError_t launch_logits_topk(float* logits, uint16_t* xb, const float* x, int64
 }
 
 hipError_t launch_logits_topk_group(float* logits, uint16_t* xb, const float* x, int64_t ldx, const float* router,
-                                    int T, int E, int H, int topk, int renorm, int32_t* ids32, float* wts, int bm,
+                                    int T, int E, int H, int topk, int renorm, int32_t* ids32, float* wts,
                                     const GroupTables& g, int32_t* hist, hipStream_t s) {
   if (T <= 0) return hipSuccess;
   const hipError_t e = launch_logits_topk(logits, xb, x, ldx, router, T, E, H, topk, renorm, ids32, wts, hist, s);
   if (e != hipSuccess) return e;
   const int blocks = fused_route_blocks(T);
-  UOCR_LAUNCH("group_scatter", k_group_scatter_hist, dim3(blocks), dim3(256), 0, s, ids32, T, E, topk, bm, blocks,
+  UOCR_LAUNCH("group_scatter", k_group_scatter_hist, dim3(blocks), dim3(256), 0, s, ids32, T, E, topk, blocks,
               kFusedTokens, hist, g);
   return hipGetLastError();
 }

@@ -108,6 +108,7 @@ hipError_t launch_rows_dense(const GemvArgs& a, hipStream_t s);
 // logits kernel and a top-k launch, else logits and top-k in one: int8 layer of
 // 1024 tokens 138 against 132 us, of 1531 186 against 190.
 constexpr int kRingTokens = 1400;
+inline bool ring_router(int T, int E, int H) { return H == 1280 && E == 64 && T >= kRingTokens; }
 // logits[t*E + e] = dot(x[t], router[e]) in the 64-lane tree order; xb (may
 // be null) receives x rounded to bf16, [T][H] (needs H % 64 == 0, H <= 2048).
 // zero (may be null): nzero words the launch clears for a later kernel.
@@ -122,21 +123,20 @@ struct GroupTables {
   int32_t* group_expert;  // [E]
   int32_t* group_start;   // [E + 1]
   int32_t* group_rows;    // [R]
-  int32_t* tile_start;    // [E + 1] prefix of ceil(count / bm), may be null
   int32_t* inv;           // [R] position of row r in group_rows, may be null
   int32_t* ctl;           // [nctl] words the prefill grouping clears for a later kernel, may be null
   int nctl;
 };
 // Groups R rows by their clamped expert id (ascending expert).
-hipError_t launch_group(const int32_t* ids, int R, int E, int bm, const GroupTables& g, hipStream_t s);
+hipError_t launch_group(const int32_t* ids, int R, int E, const GroupTables& g, hipStream_t s);
 // Prefill routing over many workgroups (E <= 64): softmax + top-k of T
 // tokens and their rows per expert in 16-token blocks, then the grouping of
 // their T*topk rows.  `hist` holds route_count_blocks(T) * E ints of scratch.
 constexpr int kRouteMaxExperts = 64;  // a lane per expert in the top-k
 int route_count_blocks(int T);
 hipError_t launch_topk_group(const float* logits, int T, int E, int topk, int renorm, int32_t* ids32, float* wts,
-                             int bm, const GroupTables& g, int32_t* hist, hipStream_t s);
-// Prefill routing for T < 2048 (E <= 64): logits, softmax + top-k and
+                             const GroupTables& g, int32_t* hist, hipStream_t s);
+// Prefill routing for T < 2048 without ring_router (E <= 64): logits, softmax + top-k and
 // per-workgroup counts in one launch (xb as launch_logits), then the
 // grouping.  hist holds fused_route_blocks(T) * E ints of scratch.
 int fused_route_blocks(int T);
@@ -146,7 +146,7 @@ hipError_t launch_logits_topk(float* logits, uint16_t* xb, const float* x, int64
                               int E, int H, int topk, int renorm, int32_t* ids32, float* wts, int32_t* hist,
                               hipStream_t s);
 hipError_t launch_logits_topk_group(float* logits, uint16_t* xb, const float* x, int64_t ldx, const float* router,
-                                    int T, int E, int H, int topk, int renorm, int32_t* ids32, float* wts, int bm,
+                                    int T, int E, int H, int topk, int renorm, int32_t* ids32, float* wts,
                                     const GroupTables& g, int32_t* hist, hipStream_t s);
 // Decode-size routing in one workgroup: softmax + top-k of T <= 64 tokens, then
 // the grouping of their T*topk rows.
@@ -181,7 +181,6 @@ struct GemmProblem {
   int N, K, groups;
   // rows
   Rows rows;
-  const int32_t* tile_start;  // [max_groups + 1] m-tile prefix (routed), null for dense
   int max_groups;
   int M;                      // dense rows (identity); routed: the rows of all groups (bounds the tiles)
   // output

@@ -337,13 +337,12 @@ int waves_for(int nchunks) {
 
 int batch_for(int nchunks) { return nchunks < kGemvMaxBatch ? (nchunks < 1 ? 1 : nchunks) : kGemvMaxBatch; }
 
-GroupTables carve_tables(Carve& c, int E, int R, bool tiles, bool inv) {
+GroupTables carve_tables(Carve& c, int E, int R, bool inv) {
   GroupTables g{};
   g.n_groups = c.take<int32_t>(1);
   g.group_expert = c.take<int32_t>(E);
   g.group_start = c.take<int32_t>(E + 1);
   g.group_rows = c.take<int32_t>(R > 0 ? R : 1);
-  g.tile_start = tiles ? c.take<int32_t>(E + 1) : nullptr;
   g.inv = inv ? c.take<int32_t>(R > 0 ? R : 1) : nullptr;
   return g;
 }
@@ -361,12 +360,12 @@ int routed_qmv(const char* op, WKind kind, float* result, const float* x, const 
     return fail(err, errlen, "%s: dimensions beyond 2^30 are not supported", op);
   const int max_groups = (int)(E < k ? E : k);
   Carve dry(nullptr);
-  carve_tables(dry, (int)E, (int)k, false, false);
+  carve_tables(dry, (int)E, (int)k, false);
   void* ws = nullptr;
   if (resolve_workspace(op, nullptr, 0, dry.off, s, &ws, err, errlen)) return 1;
   Carve c(ws);
-  const GroupTables g = carve_tables(c, (int)E, (int)k, false, false);
-  hipError_t e = launch_group(ids, (int)k, (int)E, 1, g, s);
+  const GroupTables g = carve_tables(c, (int)E, (int)k, false);
+  hipError_t e = launch_group(ids, (int)k, (int)E, g, s);
   if (e != hipSuccess) return hip_fail(err, errlen, op, e);
 
   GemvArgs a{};
@@ -813,7 +812,7 @@ static DecodeBufs carve_decode(Carve& c, const uocr_moe_layer* L, int64_t B) {
   d.logits = c.take<float>(B * L->num_experts);
   d.ids = c.take<int32_t>(R);
   d.wts = c.take<float>(R);
-  d.g = carve_tables(c, (int)L->num_experts, (int)R, false, false);
+  d.g = carve_tables(c, (int)L->num_experts, (int)R, false);
   d.h = c.take<float>(R * L->ffn);
   d.hs = c.take<float>(B * L->shared_ffn);
   d.y = c.take<float>(R * L->hidden);
@@ -941,12 +940,12 @@ static PrefillBufs carve_prefill(Carve& c, const uocr_moe_layer* L, int64_t T) {
   d.logits = c.take<float>(T * L->num_experts);
   d.ids = c.take<int32_t>(R);
   d.wts = c.take<float>(R);
-  d.g = carve_tables(c, (int)L->num_experts, (int)R, true, true);
+  d.g = carve_tables(c, (int)L->num_experts, (int)R, true);
   d.hb = c.take<uint16_t>(R * L->ffn);
   d.hsb = c.take<uint16_t>(T * L->shared_ffn);
   d.y = c.take<float>(R * L->hidden);
   d.sh = c.take<float>(2 * T * L->hidden);  // the shared experts' down sums, in up to two K ranges
-  // (the T < 2048 routing's 4-token blocks outnumber the T >= 2048 one's 16-token blocks)
+  // (the 4-token blocks of the one-launch logits and top-k outnumber the 16-token blocks of the two)
   d.hist = c.take<int32_t>((int64_t)fused_route_blocks((int)T) * L->num_experts);
   d.g.nctl = moe_layer_ctl_words(T);
   d.g.ctl = c.take<int32_t>(d.g.nctl);
@@ -1313,7 +1312,6 @@ int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden, co
   if (seq == 0) return 0;
   const hipStream_t s = (hipStream_t)stream;
   const int64_t T = seq, R = seq * L->top_k;
-  const int BM = R >= 8192 && vec ? 128 : 64;  // rows per GEMM tile
   Carve dry(nullptr);
   carve_prefill(dry, L, T);
   void* ws = nullptr;
@@ -1322,17 +1320,17 @@ int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden, co
   const PrefillBufs d = carve_prefill(c, L, T);
   const int E = (int)L->num_experts, H = (int)L->hidden, F = (int)L->ffn, Fs = (int)L->shared_ffn;
 
-  // routing (E <= 64 here): below 2048 tokens (kRingTokens for the served router) one launch computes the logits, the top-k and
-  // per-workgroup counts; above, the logits tiles share router rows over more tokens and the
-  // top-k runs in its own launch
+  // routing (E <= 64 here): below 2048 tokens (kRingTokens for the served router) one launch computes the
+  // logits, the top-k and per-workgroup counts; above, the logits tiles share router rows over more tokens
+  // and the top-k runs in its own launch
   hipError_t e = hipSuccess;
-  if (T < (H == 1280 && E == 64 ? kRingTokens : 2048)) {
+  if (T < 2048 && !ring_router((int)T, E, H)) {
     e = launch_logits_topk_group(d.logits, d.xb, x, H, L->router, (int)T, E, H, (int)L->top_k, L->renormalize, d.ids,
-                                 d.wts, BM, d.g, d.hist, s);
+                                 d.wts, d.g, d.hist, s);
   } else {
     e = launch_logits(d.logits, x, H, L->router, (int)T, E, H, d.xb, s);
     if (e == hipSuccess)
-      e = launch_topk_group(d.logits, (int)T, E, (int)L->top_k, L->renormalize, d.ids, d.wts, BM, d.g, d.hist, s);
+      e = launch_topk_group(d.logits, (int)T, E, (int)L->top_k, L->renormalize, d.ids, d.wts, d.g, d.hist, s);
   }
   if (e != hipSuccess) return hip_fail(err, errlen, op, e);
   const int max_groups = (int)(E < R ? E : R);
@@ -1349,7 +1347,6 @@ int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden, co
   gu.K = H;
   gu.groups = L->int8 ? (int)(H / L->group) : 1;
   gu.rows = rows_of(d.g);
-  gu.tile_start = d.g.tile_start;
   gu.max_groups = max_groups;
   gu.M = (int)R;
   gu.swiglu = 1;
