@@ -1,11 +1,12 @@
 """The grouped GEMM's tile placements, restated on the CPU: every tile of a launch is run exactly once.
 
-``csrc/gemm.hip`` places a launch's tiles two ways (``walk_balanced`` and ``walk_classes``); a tile
-placed twice would be computed twice (the same bits, so no output test notices the waste), and a tile
-placed nowhere would leave its rows unwritten.  This restates the balanced placement's arithmetic --
+``csrc/gemm.hip`` lists a launch's tiles per XCD in two ways (``walk_balanced`` and ``walk_classes``); a tile
+listed twice would be computed twice (the same bits, so no output test notices the waste), and a tile
+listed nowhere would leave its rows unwritten.  This restates the balanced placement's arithmetic --
 the groups ranked by rows (``make_seq``), the routed sequence cut into 8 equal-cost ranges
-(``seq_below``, ``group_below``, ``below``), the shared row tiles in 8 runs, and each workgroup's walk
-(``walk_of``: two rounds, the second reversed, or rounds in order) -- and checks, for skewed and
+(``seq_below``, ``group_below``, ``below``), the shared row tiles in 8 runs -- and each workgroup's walk of
+its XCD's list in a phase alone (``walk``: two rounds, the second reversed, or rounds in order; with both
+phases in one launch a list's tiles are taken by ticket, in order and each once) -- and checks, for skewed and
 adversarial routings and the served shapes, that the walks of all 8 x 64 workgroups cover every tile
 of both problems exactly once with rows inside the tile's group.  Planted mistakes (shared runs of
 rtb // 8 row tiles each, which drop the remainder; the second round not reversed) must fail it.

@@ -143,3 +143,36 @@ def test_routed_ops_at_the_edges_of_the_rule(oracle, kind, e, n_, rows, kernel) 
         got, want = n(ops.moe_bf16_qmv(t(x), t(ids), t(w))), oracle.moe_bf16_qmv_chunked(x, ids, w)
     assert kernel in [name for name, _ in _lib.timing_end(8)]
     assert bits_equal(got, want)
+
+
+@pytest.mark.parametrize("value", [1e-41, np.inf, np.nan], ids=["denormal", "inf", "nan"])
+def test_special_weights_and_scales(oracle, value) -> None:
+    """A denormal, infinite or NaN weight (bf16) or scale (int8) stays in its own column, with the chain's bits."""
+    from uocr_moe import ops
+
+    rng = np.random.default_rng(11)
+    x = rng.standard_normal((12, 256)).astype(np.float32)
+    col = 37
+
+    def same(got, want) -> None:
+        other = np.arange(got.shape[1]) != col
+        assert bits_equal(got[:, other], want[:, other])
+        nan = np.isnan(want[:, col])
+        assert np.array_equal(np.isnan(got[:, col]), nan)
+        assert bits_equal(got[~nan][:, [col]], want[~nan][:, [col]])
+
+    dense = rng.standard_normal((16, 80, 16)).astype(np.float32)
+    dense[3, col, 5] = value
+    dense = oracle.bf16_bits(dense)
+    same(n(ops.dense_bf16_qmv(t(x), t(dense))), oracle.dense_bf16_qmv_chunked(x, dense))
+    ids = np.zeros(12, np.int32)
+    rows = rng.standard_normal((1, 80, 256)).astype(np.float32)
+    rows[0, col, 200] = value
+    rows = oracle.bf16_bits(rows)
+    same(n(ops.moe_bf16_qmv(t(x), t(ids), t(rows))), oracle.moe_bf16_qmv_chunked(x, ids, rows))
+    # int8: wide enough for the matrix kernel
+    ids = np.arange(12, dtype=np.int32)
+    w = rng.integers(-127, 128, (12, 704, 256)).astype(np.int8)
+    s = rng.uniform(1e-4, 1e-2, (12, 704, 2)).astype(np.float32)
+    s[:, col, 1] = value
+    same(n(ops.moe_int8_qmv(t(x), t(ids), t(w), t(s))), oracle.moe_int8_qmv(x, ids, w, s))

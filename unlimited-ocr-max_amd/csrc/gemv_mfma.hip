@@ -5,7 +5,8 @@
 // one fma chain in ascending k from 0, the chunks folded in order.  One
 // 4x4x1 instruction is 16 blocks of 4 x 4 outputs, D = A B + C with K = 1:
 // each output takes one fused multiply-add, rounded as fmaf rounds it
-// (denormals kept; checked against fmaf over all bit patterns), so a series
+// (denormals kept; the tests compare bits with the oracle's fmaf chains, with
+// denormal, infinite and NaN rows, weights and scales among them), so a series
 // of them over k is the chain.  Block b's 4 columns are lanes 4b .. 4b + 3 of
 // the B operand, so B is "lane = output column" and D's register r is row r:
 // the layout of the VALU kernel.  The A operand broadcasts one block (cbsz
@@ -20,9 +21,11 @@
 // k takes 7 ns for up to 4 rows, 9 for 8, 13 for 12, 16 for 16; the waves of a
 // SIMD take turns).  Against the VALU kernel: 37 int8 decode rows, gate/up 224
 // -> 47 us (156 MB; 33 us with the chains left out, 45 with the loads left
-// out) and down 157 -> 26 us; lm_head (331 MB) at 1 / 8 / 64 rows 67 / 85 /
-// 658 -> 54 / 57 / 205 us; q/k/v at 1 / 8 / 20 rows 6.1 / 13.1 / 30.9 -> 4.4 /
-// 5.9 / 8.6 us; the 6848-wide down at 8 rows 58 -> 10.4 us.
+// out) and down 157 -> 26 us; lm_head (331 MB) at 2 / 8 / 64 rows 69 / 84 /
+// 662 -> 58 / 58 / 207 us; q/k/v at 1 / 8 / 64 rows 6.5 / 13.5 / 88 -> 5.2 /
+// 6.8 / 14 us; the 6848-wide down at 8 rows 59 -> 11 us.  A layer's pair of
+// launches at any number of rows, also 1: hidden 4096, ffn 1408, 64 experts, 1
+// / 8 int8 rows 145 / 565 -> 90 / 176 us.
 #include "uocr_device.h"
 #include "uocr_kernels.h"
 
