@@ -299,3 +299,24 @@ def test_graph_replays_match_eager() -> None:
             assert np.array_equal(n(outs[layer]).view(np.uint32), eager[layer].view(np.uint32)), (rep, layer)
         run()  # eager work between the replays
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("lengths", [[900, 700, 512, 1], [1, 130, 1024, 257, 640, 128, 129, 896]])
+def test_a_wide_table_gives_the_same_rows(lengths) -> None:
+    """More than 65535 splits, all but a few of them empty, against the launch of the attended ones."""
+    uocr = _ops()
+    g = torch.Generator(device="cuda:0").manual_seed(5)
+    rows, heads, page = len(lengths), 1, 128
+    per = -(-max(lengths) // page)
+    pages = rows * per + 1
+    pool = torch.randn((pages, 2, 1, page, heads, D), generator=g, device="cuda:0")
+    q, k, v = (torch.randn((rows, heads, D), generator=g, device="cuda:0") for _ in range(3))
+    last = torch.tensor([a - 1 for a in lengths], dtype=torch.int32, device="cuda:0")
+    got = []
+    for cols in (per, 65537):
+        table = torch.full((rows, cols), pages - 1, dtype=torch.int32, device="cuda:0")
+        table[:, :per] = torch.arange(rows * per, device="cuda:0", dtype=torch.int32).view(rows, per)
+        kv = uocr.PagedKv(kv_blocks=pool.clone(), lookup_table=table, attend_lengths=last,
+                          attend_max=cols * page, write_index=last)
+        got.append((n(uocr.paged_decode_attention(q, k, v, kv=kv, layer_idx=0, scale=SCALE)), n(kv.kv_blocks)))
+    assert all(np.array_equal(a.view(np.uint32), b.view(np.uint32)) for a, b in zip(*got))

@@ -60,6 +60,7 @@ struct PagedArgs {
   const float* cos_t;
   const float* sin_t;
   int table_rows;
+  int split_x;  // the grid is (splits, heads, rows), else (heads, rows, splits)
 };
 
 // RoPE of the pair (x[d], x[d + 64]) with cos / sin rows c, s: each product
@@ -161,8 +162,8 @@ __device__ __forceinline__ void split_partial(const PagedArgs& a, const float* _
   // attended ones' loads (no branch, and no bytes of rows that are not attended); their values are
   // masked below.  The step's metadata and the pool row's address are read in one round trip, q's
   // tables before the keys.  Against reading whole splits, a round trip more (cold pages, us): 1 row of
-  // 16 / 128 / 640 6.4 -> 5.5, 6.9 -> 7.1, 8.4 -> 8.5; 8 rows of 300 / 640 / 1200 11.1 -> 9.9, 16.4 ->
-  // 16.3, 27.8 -> 26.5.  (Lanes that all repeat the last row: 1 row of 16 5.9.)
+  // 16 / 128 / 640 6.4 -> 5.5, 6.9 -> 7.1, 8.4 -> 8.6; 8 rows of 300 / 640 / 1200 11.1 -> 9.9, 16.4 ->
+  // 16.4, 27.8 -> 26.3.  (Lanes that all repeat the last row: 1 row of 16 5.9.)
   const int n = r1 - r0;
   const int sub = tid % kLanesPerRow, rg = tid / kLanesPerRow;
   const int c = tid % (kD / 4), g = tid / (kD / 4);
@@ -305,7 +306,8 @@ __global__ void __launch_bounds__(kThreads, 4) k_attn_partial(PagedArgs a, const
   __shared__ float red[kThreads / 64];
   __shared__ f32x4 vsum[kValueGroups - 1][kD / 4];
   __shared__ uint32_t last;
-  const int s = (int)blockIdx.x, h = (int)blockIdx.y, b = (int)blockIdx.z;
+  const int s = (int)(a.split_x ? blockIdx.x : blockIdx.z), h = (int)(a.split_x ? blockIdx.y : blockIdx.x);
+  const int b = (int)(a.split_x ? blockIdx.z : blockIdx.y);
   const int tid = (int)threadIdx.x;
   const int r0 = s * kAttnSplitRows;
   // Device metadata (one memory round trip), clamped to what the lookup row addresses (never out of the pool).
@@ -386,9 +388,14 @@ hipError_t launch_paged_attention(const PagedAttention& p, hipStream_t s) {
   a.sin_t = p.sin_table;
   a.table_rows = p.table_rows;
   const int splits = (p.max_attend + kAttnSplitRows - 1) / kAttnSplitRows;
-  // (The heads of a split side by side, neighbours in memory, took 0.2 us more at 1 row and 0.4 at 8 of 640.)
+  // Splits outermost: every request's first splits start first and all XCDs share them.  Side by side, a
+  // split's workgroups shared an XCD where there are 8 splits, and those of the last ones idled behind shorter
+  // requests (8 rows of up to 900 / 1280: 17.9, 24.2 us with a request's splits and heads together, 18.7, 23.9
+  // with its splits together, 17.2, 21.9 so; of up to 640 13.4, 12.7, 13.3).  More than 65535 splits go to the dimension that holds them.
   const int ns = splits > 0 ? splits : 1;
-  const dim3 grid((unsigned)ns, (unsigned)p.heads, (unsigned)p.rows);
+  a.split_x = ns > 65535;
+  const dim3 grid = a.split_x ? dim3((unsigned)ns, (unsigned)p.heads, (unsigned)p.rows)
+                              : dim3((unsigned)p.heads, (unsigned)p.rows, (unsigned)ns);
   UOCR_LAUNCH("attn_partial", k_attn_partial, grid, dim3(kThreads), 0, s, a, p.q, p.k_new, p.v_new, p.scale,
               p.workspace, ns, p.counters, p.out);
   if (ns > 1 && p.counters == nullptr)
