@@ -388,12 +388,14 @@ hipError_t launch_paged_attention(const PagedAttention& p, hipStream_t s) {
   a.sin_t = p.sin_table;
   a.table_rows = p.table_rows;
   const int splits = (p.max_attend + kAttnSplitRows - 1) / kAttnSplitRows;
-  // Splits outermost: every request's first splits start first and all XCDs share them.  Side by side, a
-  // split's workgroups shared an XCD where there are 8 splits, and those of the last ones idled behind shorter
-  // requests (8 rows of up to 900 / 1280: 17.9, 24.2 us with a request's splits and heads together, 18.7, 23.9
-  // with its splits together, 17.2, 21.9 so; of up to 640 13.4, 12.7, 13.3).  More than 65535 splits go to the dimension that holds them.
+  // A request's splits side by side where their number is odd, so that they go round the XCDs; else splits
+  // outermost.  With an even number side by side a split's workgroups share few XCDs (8 splits: one), and those
+  // of the last splits idle behind shorter requests.  8 rows of up to 900 / 1280 (8, 10 splits): 18.6, 23.7 us
+  // side by side, 17.2, 21.8 so; of up to 640 / 1150 (5, 9): 12.5, 21.4 side by side, 13.2, 20.6 outermost.  (A
+  // split's heads together, then the splits: 13.1, 17.8, 22.2, 24.1.)  More than 65535 splits go to the
+  // dimension that holds them.
   const int ns = splits > 0 ? splits : 1;
-  a.split_x = ns > 65535;
+  a.split_x = ns % 2 != 0 || ns > 65535;
   const dim3 grid = a.split_x ? dim3((unsigned)ns, (unsigned)p.heads, (unsigned)p.rows)
                               : dim3((unsigned)p.heads, (unsigned)p.rows, (unsigned)ns);
   UOCR_LAUNCH("attn_partial", k_attn_partial, grid, dim3(kThreads), 0, s, a, p.q, p.k_new, p.v_new, p.scale,

@@ -1402,8 +1402,9 @@ int uocr_moe_forward(float* out, const float* x, int64_t seq, int64_t hidden, co
   sdn.kparts = gemm_shared_parts(dn, sdn);
   sdn.part_stride = T * H;
   // One launch: its down tiles read h past the L2, once for each of hidden / 256 column tiles.  Up to 8 that
-  // costs less than a second launch (bf16, T = 4096, hidden 1280 / 2048: 421 / 997 us against 434 / 1003),
-  // beyond it costs more (hidden 3072 / 4096, ffn 1408: 1727 / 2265 against 1520 / 2037).
+  // costs less than a second launch or about as much (us with one, two: hidden 1280 bf16, T = 1531 / 4096 223,
+  // 250 / 421, 434; hidden 2048, ffn 1408, T = 4096 int8 775, 820, bf16 997, 957), beyond it costs more (bf16,
+  // T = 4096, hidden 3072 / 4096, ffn 1408 1727, 1520 / 2265, 2037).
   const bool staged = vec && aligned16(ws);
   if (H <= 2048 && gemm_staged_ok(gu, staged) && gemm_staged_ok(dn, staged)) {
     e = launch_moe_layer(gu, sgu, dn, sdn, d.g.ctl, spin_limit(kPrefillSpin), d.wts, (int)R, s);
